@@ -589,7 +589,7 @@ int hip_add_rmsnorm_q8k(const float *h, const float *delta, const float *w, floa
     if (rc) return rc;
     if (!h || !w) return fail(QK_ERR_ARG, "null pointer");
     if (!x_out && !xq) return fail(QK_ERR_ARG, "x_out and xq are both NULL");
-    // one 256-thread workgroup per row; a dispatch counts work-items in 32 bits
+    // one workgroup of a thread per four elements (at least 64) per row; a dispatch counts work-items in 32 bits
     if (m < 1 || m >= ((int64_t)1 << 24) || k < 4 || k % 4 || k > QK_NORM_MAX_K)
         return fail(QK_ERR_ARG, "bad shape m=%lld k=%lld (m below 2^24, k a multiple of 4, at most %d)",
                     (long long)m, (long long)k, QK_NORM_MAX_K);

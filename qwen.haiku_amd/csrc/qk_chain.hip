@@ -22,33 +22,21 @@ __device__ __forceinline__ float silu(float v) {
 
 // ---- the norm's sequential double sum ----------------------------------
 // tensor_rms_norm adds (double)(r_i * r_i) to a double in index order
-// (slm/tensor.c:357-360), rounding after every add. The terms are
-// non-negative, so while every partial sum of a block of terms (and the
-// running sum s before it) is a multiple of 2^g and below 2^(g + 53), no
-// add rounds and the block's sequential sum is s + (the exact block sum),
-// computed in any order. Each block of NB_T terms therefore gets its sum
-// (in a tree), the lowest set bit over its terms and a flag for inf/NaN
-// terms in parallel; one lane then walks the blocks in order and adds a
-// block in one step when T = s + sum and g = floor(log2 T) + 2 - 53 pass
-// the test (T is within a relative 2^-46 of the true total, so the true
-// total is below 2^(g + 53) whenever T is below 2^(g + 52)), else adds
-// the block's terms one by one as the reference does.
-constexpr int NB_T = 64;                               // terms per block (one wave)
-constexpr int NB_MAX = QK_NORM_MAX_K / NB_T;
-
-// Exponent of the lowest set bit of a finite double v > 0.
-__device__ __forceinline__ int low_bit(double v) {
-    const uint64_t b = (uint64_t)__double_as_longlong(v);
-    const int e = (int)(b >> 52) & 0x7ff;
-    const uint64_t m = (b & 0xfffffffffffffull) | (e ? 0x10000000000000ull : 0);
-    return (e ? e : 1) - 1075 + __builtin_ctzll(m);
-}
-
-template <int CTRL>
+// (slm/tensor.c:357-360), rounding after every add. The chain of k adds is
+// cut into segments of four terms, one per lane. Every segment's start is
+// guessed (a scan of the segment sums, whose roundings differ from the
+// chain's now and then), every lane runs its own four adds from its guess,
+// and the guesses are checked: the first segment's start (0) is right, and
+// a segment whose start is right ends right, so when each end equals the
+// next start bit for bit the last end is the chain's. At the first end that
+// differs, the next start takes it and the later guesses move by the same
+// difference; every such step fixes at least one more segment, so the loop
+// ends for any input (infinities and NaN included).
+template <int CTRL, int ROWS = 0xF>
 __device__ __forceinline__ double dpp64(double v) {
     const uint64_t b = (uint64_t)__double_as_longlong(v);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)b, CTRL, 0xF, 0xF, true);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(b >> 32), CTRL, 0xF, 0xF, true);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, ROWS, 0xF, true);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, ROWS, 0xF, true);
     return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
 }
 
@@ -59,145 +47,151 @@ __device__ __forceinline__ double readlane64(double v, int l) {
     return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
 }
 
-// Sum over the wave (order irrelevant: used only where it is exact).
-__device__ __forceinline__ double wave_sum64(double v) {
-    v = __dadd_rn(v, dpp64<0xB1>(v));                 // quad_perm [1,0,3,2]
-    v = __dadd_rn(v, dpp64<0x4E>(v));                 // quad_perm [2,3,0,1]
-    v = __dadd_rn(v, dpp64<0x141>(v));                // row_half_mirror
-    v = __dadd_rn(v, dpp64<0x140>(v));                // row_mirror
-    return __dadd_rn(__dadd_rn(readlane64(v, 0), readlane64(v, 16)),
-                     __dadd_rn(readlane64(v, 32), readlane64(v, 48)));
+// Inclusive sums over the lanes (lanes past a row boundary get the row
+// totals before them by row_bcast). Only the first 16 lanes if `one_row`.
+__device__ __forceinline__ double wave_scan64(double v, bool one_row) {
+    v = __dadd_rn(v, dpp64<0x111>(v));                // row_shr:1
+    v = __dadd_rn(v, dpp64<0x112>(v));                // row_shr:2
+    v = __dadd_rn(v, dpp64<0x114>(v));                // row_shr:4
+    v = __dadd_rn(v, dpp64<0x118>(v));                // row_shr:8
+    if (!one_row) {
+        v = __dadd_rn(v, dpp64<0x142, 0xA>(v));       // row_bcast:15 into rows 1 and 3
+        v = __dadd_rn(v, dpp64<0x143, 0xC>(v));       // row_bcast:31 into rows 2 and 3
+    }
+    return v;
 }
 
-__device__ __forceinline__ int wave_min_i(int v) {
-    v = min(v, __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, true));
-    v = min(v, __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, true));
-    v = min(v, __builtin_amdgcn_mov_dpp(v, 0x141, 0xF, 0xF, true));
-    v = min(v, __builtin_amdgcn_mov_dpp(v, 0x140, 0xF, 0xF, true));
-    return min(min(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
-               min(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+__device__ __forceinline__ bool same_bits(double a, double b) {
+    return __double_as_longlong(a) == __double_as_longlong(b);
+}
+
+// The guesses after segment f (lanes above f) once f's end is known.
+__device__ __forceinline__ double move_starts(double st, double end, int f, int lane) {
+    const double was = readlane64(st, f + 1), by = __dsub_rn(end, was);
+    const bool finite = fabs(by) <= 1.0e308;
+    const double moved = finite ? __dadd_rn(st, by) : end;
+    return lane <= f ? st : (lane == f + 1 ? end : moved);
+}
+
+// One wave's block of 256 terms from `start`: lane l adds its terms t0 .. t3
+// after lanes 0 .. l - 1. q: the exclusive sums of the lanes before. Returns
+// the block's end (of the last lane), exact for that start.
+__device__ __forceinline__ double block_chain(double start, double q, double t0, double t1, double t2, double t3,
+                                              int lane) {
+    double st = lane == 0 ? start : __dadd_rn(start, q);
+    for (;;) {
+        const double e = __dadd_rn(__dadd_rn(__dadd_rn(__dadd_rn(st, t0), t1), t2), t3);
+        const double next = dpp64<0x130>(st);         // wave_shl:1
+        const uint64_t off = __ballot(lane < 63 && !same_bits(e, next));
+        if (off == 0) return readlane64(e, 63);
+        const int f = __builtin_ctzll(off);
+        st = move_starts(st, readlane64(e, f), f, lane);
+    }
 }
 
 // tensor_add (slm/tensor.c:284-291) of an optional delta, then
 // tensor_rms_norm (slm/tensor.c:345-367) of the sum, then optionally
-// quantize_row_q8_K (slm/tensor.c:683-720) of the normalized row. One
-// workgroup of 256 per row of k floats; the row sits in LDS (k * 4 bytes
-// of dynamic LDS).
+// quantize_row_q8_K (slm/tensor.c:683-720) of the normalized row:
 //   r      = h + delta                      (stored to h_out if given)
-//   ssq    = sum over i of (double)(r_i * r_i), the sequential double
-//            sum in index order (exact blocks in one step, see above)
+//   ssq    = sum over i of (double)(r_i * r_i), in index order (see above)
 //   rscale = 1 / sqrtf((float)(ssq / k) + eps)
 //   x_i    = (r_i * rscale) * w_i           (stored to x_out if given)
-__global__ __launch_bounds__(256) void k_add_rmsnorm(const float *h, const float *__restrict__ delta,
-                                                     const float *__restrict__ w, float eps, int64_t k,
-                                                     float *h_out, float *__restrict__ x_out,
-                                                     uint8_t *__restrict__ xq) {
-    extern __shared__ float4 row4[];                   // k / 4 float4
-    __shared__ float rscale_s;
-    const int64_t t = blockIdx.x;
-    const int64_t k4 = k >> 2;
-    const float4 *h4 = reinterpret_cast<const float4 *>(h + t * k);
-    const float4 *d4 = delta ? reinterpret_cast<const float4 *>(delta + t * k) : nullptr;
-    float4 *ho4 = h_out ? reinterpret_cast<float4 *>(h_out + t * k) : nullptr;
-    for (int64_t i = threadIdx.x; i < k4; i += 256) {
-        float4 v = h4[i];
-        if (d4) {
-            const float4 a = d4[i];
-            v.x = __fadd_rn(v.x, a.x);
-            v.y = __fadd_rn(v.y, a.y);
-            v.z = __fadd_rn(v.z, a.z);
-            v.w = __fadd_rn(v.w, a.w);
-        }
-        row4[i] = v;
-        if (ho4) ho4[i] = v;
-    }
-    __syncthreads();
-    __shared__ double bsum[NB_MAX];
-    __shared__ int blow[NB_MAX];                       // lowest set bit; INT_MIN: an inf/NaN term
-    const float *rowf = reinterpret_cast<const float *>(row4);
-    const int nblk = (int)((k + NB_T - 1) / NB_T);
+// One workgroup per row; wave v owns the 256-element blocks v, v + W, ...
+// (W waves, NB blocks each), four consecutive elements per lane, kept in
+// registers from the loads (h, delta and w all in flight at once) to the
+// stores. What bounds a decode row is latency: one round of loads, two
+// barriers (block totals; block ends), one division and square root.
+// Against one lane walking the squares in blocks of 64 (a block whose adds
+// round went term by term): 1 x 1024 5.80 -> 2.80 us a launch, 512 x 1024
+// 12.9 -> 4.9 us.
+template <int NB>
+__global__ __launch_bounds__(1024) void k_add_rmsnorm(const float *h, const float *delta,
+                                                      const float *__restrict__ w, float eps, int k, float *h_out,
+                                                      float *x_out, uint8_t *__restrict__ xq) {
+    __shared__ double total[QK_NORM_MAX_K / QK_K], ends[QK_NORM_MAX_K / QK_K];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, W = blockDim.x >> 6;
+    const int nblk = (k + QK_K - 1) / QK_K;
+    const int64_t row = (int64_t)blockIdx.x * k;
+    float4 r[NB], g[NB];
     {
-        const int lane = threadIdx.x & 63;
-        for (int b = threadIdx.x >> 6; b < nblk; b += 4) {   // one wave per block
-            const int64_t i = (int64_t)b * NB_T + lane;
-            const float x = i < k ? rowf[i] : 0.0f;
-            const double t = (double)__fmul_rn(x, x);
-            const bool special = !(t <= 1.0e308);      // inf or NaN
-            const int lb = (t > 0.0 && !special) ? low_bit(t) : 0x7fffffff;
-            const double sb = wave_sum64(special ? 0.0 : t);
-            const int lbm = wave_min_i(lb);
-            const bool any_special = __ballot(special) != 0;   // the whole wave votes
-            if (lane == 0) {
-                bsum[b] = sb;
-                blow[b] = any_special ? (int)0x80000000 : lbm;
+        float4 a[NB];
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            const int i = (wave + W * b) * QK_K + 4 * lane;
+            r[b] = a[b] = g[b] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (i < k) {                              // k is a multiple of 4
+                r[b] = *reinterpret_cast<const float4 *>(h + row + i);
+                if (delta) a[b] = *reinterpret_cast<const float4 *>(delta + row + i);
+                g[b] = *reinterpret_cast<const float4 *>(w + i);
             }
         }
+        if (delta)
+#pragma unroll
+            for (int b = 0; b < NB; b++)
+                r[b] = make_float4(__fadd_rn(r[b].x, a[b].x), __fadd_rn(r[b].y, a[b].y), __fadd_rn(r[b].z, a[b].z),
+                                   __fadd_rn(r[b].w, a[b].w));
+    }
+    double t[NB][4], q[NB];
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+        const int i = (wave + W * b) * QK_K + 4 * lane;
+        if (h_out && i < k) *reinterpret_cast<float4 *>(h_out + row + i) = r[b];
+        t[b][0] = (double)__fmul_rn(r[b].x, r[b].x);
+        t[b][1] = (double)__fmul_rn(r[b].y, r[b].y);
+        t[b][2] = (double)__fmul_rn(r[b].z, r[b].z);
+        t[b][3] = (double)__fmul_rn(r[b].w, r[b].w);
+        const double own = __dadd_rn(__dadd_rn(t[b][0], t[b][1]), __dadd_rn(t[b][2], t[b][3]));
+        const double incl = wave_scan64(own, false);
+        q[b] = dpp64<0x138>(incl);                    // wave_shr:1
+        if (lane == 63 && wave + W * b < nblk) total[wave + W * b] = incl;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double ssq = 0.0;
-        for (int b = 0; b < nblk; b++) {
-            const double T = __dadd_rn(ssq, bsum[b]);
-            bool exact = blow[b] != (int)0x80000000;
-            if (exact && T > 0.0) {
-                const int g = (int)(((uint64_t)__double_as_longlong(T) >> 52) & 0x7ff) - 1023 + 2 - 53;
-                exact = blow[b] >= g && (ssq == 0.0 || low_bit(ssq) >= g);
-            }
-            if (exact) {
-                ssq = T;                                // every add of the block was exact
-                continue;
-            }
-            // the block one term at a time: its float4s read first, then
-            // the dependent adds (k is a multiple of 4)
-            const int64_t q0 = (int64_t)b * (NB_T / 4);
-            auto add4 = [&](const float4 v) {
-                ssq = __dadd_rn(ssq, (double)__fmul_rn(v.x, v.x));
-                ssq = __dadd_rn(ssq, (double)__fmul_rn(v.y, v.y));
-                ssq = __dadd_rn(ssq, (double)__fmul_rn(v.z, v.z));
-                ssq = __dadd_rn(ssq, (double)__fmul_rn(v.w, v.w));
-            };
-            if (q0 + NB_T / 4 <= k4) {                  // a whole block
-                float4 v[NB_T / 4];
+    // lane b of every wave: the guessed start of block b
+    double starts = dpp64<0x138>(wave_scan64(lane < nblk ? total[lane] : 0.0, nblk <= 16));
+    double ssq;
+    for (;;) {                                        // uniform: every wave sees the same ends
 #pragma unroll
-                for (int q = 0; q < NB_T / 4; q++) v[q] = row4[q0 + q];
-#pragma unroll
-                for (int q = 0; q < NB_T / 4; q++) add4(v[q]);
-            } else {                                    // the row's last, partial block
-                for (int64_t q = q0; q < k4; q++) add4(row4[q]);
+        for (int b = 0; b < NB; b++) {
+            const int blk = wave + W * b;
+            if (blk < nblk) {
+                const double e = block_chain(readlane64(starts, blk), q[b], t[b][0], t[b][1], t[b][2], t[b][3], lane);
+                if (lane == 0) ends[blk] = e;
             }
         }
-        const float ms = __double2float_rn(__ddiv_rn(ssq, (double)k));
-        // __builtin_sqrtf is the correctly rounded square root (the raw
-        // v_sqrt_f32 that __fsqrt_rn maps to is not)
-        rscale_s = __fdiv_rn(1.0f, __builtin_sqrtf(__fadd_rn(ms, eps)));
+        __syncthreads();
+        const double e = lane < nblk ? ends[lane] : 0.0;
+        const double next = dpp64<0x130>(starts);
+        const uint64_t off = __ballot(lane < nblk - 1 && !same_bits(e, next));
+        if (off == 0) {
+            ssq = readlane64(e, nblk - 1);
+            break;
+        }
+        const int f = __builtin_ctzll(off);
+        starts = move_starts(starts, readlane64(e, f), f, lane);
+        __syncthreads();                              // the ends are rewritten
     }
-    __syncthreads();
-    const float rscale = rscale_s;
-    const float4 *w4 = reinterpret_cast<const float4 *>(w);
-    float4 *xo4 = x_out ? reinterpret_cast<float4 *>(x_out + t * k) : nullptr;
-    if (xq) {
-        // one wave per 256-element block, 4 consecutive elements per lane
-        const int lane = threadIdx.x & 63;
-        const int64_t nb = k / QK_K;
-        for (int64_t b = threadIdx.x >> 6; b < nb; b += 4) {
-            const int64_t i = b * 64 + lane;
-            const float4 v = row4[i], g = w4[i];
-            const float e[4] = {__fmul_rn(__fmul_rn(v.x, rscale), g.x), __fmul_rn(__fmul_rn(v.y, rscale), g.y),
-                                __fmul_rn(__fmul_rn(v.z, rscale), g.z), __fmul_rn(__fmul_rn(v.w, rscale), g.w)};
-            if (xo4) xo4[i] = make_float4(e[0], e[1], e[2], e[3]);
+    // ssq / k; for a power of two the product with 1 / k is the same value
+    const double mean = (k & (k - 1)) == 0 ? __dmul_rn(ssq, 1.0 / (double)k) : __ddiv_rn(ssq, (double)k);
+    // __builtin_sqrtf is the correctly rounded square root (the raw
+    // v_sqrt_f32 that __fsqrt_rn maps to is not)
+    const float rscale = __fdiv_rn(1.0f, __builtin_sqrtf(__fadd_rn(__double2float_rn(mean), eps)));
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+        const int blk = wave + W * b, i = blk * QK_K + 4 * lane;
+        if (blk >= nblk) break;                       // whole wave
+        const float e[4] = {__fmul_rn(__fmul_rn(r[b].x, rscale), g[b].x),
+                            __fmul_rn(__fmul_rn(r[b].y, rscale), g[b].y),
+                            __fmul_rn(__fmul_rn(r[b].z, rscale), g[b].z),
+                            __fmul_rn(__fmul_rn(r[b].w, rscale), g[b].w)};
+        if (x_out && i < k) *reinterpret_cast<float4 *>(x_out + row + i) = make_float4(e[0], e[1], e[2], e[3]);
+        if (xq) {                                     // k % 256 == 0: every lane is in range
             uint32_t packed, bs;
             float d;
             q8k_block_wave(e, lane, packed, d, bs);
-            uint8_t *out = xq + (t * nb + b) * Q8K_BYTES;
+            uint8_t *out = xq + ((int64_t)blockIdx.x * nblk + blk) * Q8K_BYTES;
             reinterpret_cast<uint32_t *>(out + 4)[lane] = packed;
             if ((lane & 7) == 0) reinterpret_cast<uint32_t *>(out + 260)[lane >> 3] = bs;
             if (lane == 0) *reinterpret_cast<float *>(out) = d;
-        }
-    } else {
-        for (int64_t i = threadIdx.x; i < k4; i += 256) {
-            const float4 v = row4[i], g = w4[i];
-            xo4[i] = make_float4(__fmul_rn(__fmul_rn(v.x, rscale), g.x), __fmul_rn(__fmul_rn(v.y, rscale), g.y),
-                                 __fmul_rn(__fmul_rn(v.z, rscale), g.z), __fmul_rn(__fmul_rn(v.w, rscale), g.w));
         }
     }
 }
@@ -241,10 +235,20 @@ __global__ __launch_bounds__(256) void k_swiglu(const float *__restrict__ gate, 
 }
 
 // ---- launchers ---------------------------------------------------------
+// One wave per 256-element block up to 16 waves, then several blocks each.
+// A dispatch counts its work-items in 32 bits, so more than 2^21 rows of
+// up to 1024 threads go out in several launches.
 hipError_t launch_add_rmsnorm(const float *h, const float *delta, const float *w, float eps, int64_t m, int64_t k,
                               float *h_out, float *x_out, uint8_t *xq, hipStream_t s) {
-    hipLaunchKernelGGL(k_add_rmsnorm, dim3((unsigned)m), dim3(256), (size_t)k * sizeof(float), s, h, delta, w, eps,
-                       k, h_out, x_out, xq);
+    const int nblk = (int)((k + QK_K - 1) / QK_K), waves = nblk < 16 ? nblk : 16;
+    auto kernel = nblk <= 16 ? k_add_rmsnorm<1> : nblk <= 32 ? k_add_rmsnorm<2> : k_add_rmsnorm<4>;
+    const int64_t rows = (int64_t)1 << 21;
+    for (int64_t t = 0; t < m; t += rows) {
+        const unsigned grid = (unsigned)(m - t < rows ? m - t : rows);
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * waves), 0, s, h + t * k, delta ? delta + t * k : nullptr, w,
+                           eps, (int)k, h_out ? h_out + t * k : nullptr, x_out ? x_out + t * k : nullptr,
+                           xq ? xq + t * nblk * Q8K_BYTES : nullptr);
+    }
     return hipGetLastError();
 }
 

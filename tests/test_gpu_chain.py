@@ -113,6 +113,33 @@ def test_add_rmsnorm_block_paths(lib, orc, k):
     assert_bits_equal(host(xo), orc.add_rmsnorm(h, None, w, 1e-6)[1], f"block paths k={k}")
 
 
+@pytest.mark.parametrize("k", [8, 252, 260, 4096, 4100, 8192, 8196, 16380])
+def test_add_rmsnorm_chain_splits(lib, orc, k):
+    """The widths around which the chain's split changes (one lane, a
+    partial block, one to four blocks per wave), on rows whose guessed
+    segment starts are wrong often: scales that change from element to
+    element, sums that round at every add, infinities and NaN."""
+    step(f"add_rmsnorm chain splits k={k}")
+    rng = np.random.default_rng(k + 9)
+    rows = list(norm_block_rows(k, rng))
+    for spread in (4, 12, 28):
+        rows.append(rng.standard_normal(k) * np.exp2(rng.integers(-spread, spread + 1, k)))
+    falling = np.exp2(np.linspace(30, -30, k)) * rng.uniform(1, 2, k)
+    rows += [falling, falling[::-1], np.full(k, 1.0 + 2.0 ** -12)]
+    for where in (0, k // 2, k - 1):
+        for v in (np.inf, np.nan, 3e38):
+            bad = rng.standard_normal(k)
+            bad[where] = v
+            rows.append(bad)
+    h = np.asarray(rows, np.float32)
+    w = (1 + 0.02 * rng.standard_normal(k)).astype(np.float32)
+    ho, xo = empty(h.shape), empty(h.shape)
+    lib.add_rmsnorm_q8k(dev(h), None, dev(w), 1e-6, h_out=ho, x_out=xo)
+    want_r, want_x = orc.add_rmsnorm(h, None, w, 1e-6)
+    assert_bits_equal(host(ho), want_r, "h")
+    assert_bits_equal(host(xo), want_x, f"chain splits k={k}")
+
+
 def test_add_rmsnorm_many_scales(lib, orc):
     """4096 constant rows spanning 60 binades: as many distinct
     rscale = 1/sqrtf(mean + eps) values, each correctly rounded."""
