@@ -7,24 +7,22 @@
 // The reference runs on the host with plain fp32 loops; on x86 each dot
 // and each axpy is a sequential chain of separately rounded products and
 // sums (no FMA in its build), and its result depends on that order. Here
-// every output element is one lane that runs its reduction in exactly the
-// reference's order, skipping the zero coefficients the reference skips;
-// the parallelism is across outputs, heads and chunks. There are seven
-// phases, each reading the previous phases' results from the per-(chunk,
-// head) scratch below; phases 1-4 do not depend on the carried state and
-// run for a group of chunks at once, one launch each, and phases 5-7 run
-// chunk after chunk inside one launch (this file is built with
-// -ffp-contract=off; the only fused multiply-adds are inside qk_expf):
+// every output element is one lane's chain in exactly the reference's
+// order; the parallelism is across outputs, heads and chunks (this file is
+// built with -ffp-contract=off; the only fused multiply-adds are inside
+// qk_expf). Two launches per group of chunks:
 //
-//   1 cumulative gate, exps, decay mask; K*beta, V*beta, K*beta*exp(gcs),
-//     Q*exp(gcs)
-//   2 KK^T and KQ^T scaled by the decay (tiles staged in LDS)
-//   3 forward substitution of the unit lower system, one lane per column
-//   4 attn @ V*beta, attn @ K*beta*exp(gcs)
-//   5 the carried state against Q*exp(gcs) and against the decayed keys;
-//     v_new
-//   6 the intra-chunk attention on v_new; the output rows
-//   7 state := state * exp(g_last) + (K * exp(g_last - gcs))^T v_new
+//   k_dn_chunk  what does not depend on the carried state, every (chunk,
+//               head) at once: the gates, KK^T and KQ^T with the decay, the
+//               triangular solve, attn @ V*beta and attn @ K*beta*exp(gcs)
+//   k_dn_carry  chunk after chunk: the state against Q*exp(gcs) and the
+//               decayed keys, v_new, the output rows, the state carried on
+//
+// Where the reference skips a zero coefficient, the chain adds the zero
+// product instead: a sum that starts at +0 is never -0, so adding +-0 leaves
+// it as it is. That fails only for an infinite or NaN factor, so the kernels
+// watch the factors (V*beta, K*beta*exp(gcs), the state) and take a copy of
+// the loop with the skip when one is not finite.
 #include "qk_dev.h"
 #include "qk_expf.h"
 #include "qk_kernels.h"
@@ -32,21 +30,17 @@
 namespace qk {
 
 constexpr int DN_C = 64;                               // chunk size (CHUNK_SIZE)
-constexpr int DN_D = 128;                              // largest head dim handled
+constexpr int DN_D = 128;                              // largest head dim handled; row stride of the scratch
 
-// Scratch of one group of chunks (floats), one slot per (chunk, head).
+// Scratch of one group of chunks (floats), one slot per (chunk, head). Rows
+// past the chunk and columns past the head dims hold zeros.
 struct DnScratch {
-    float *gv;      // [H][3*64 + 1]: gcs | exp(gcs) | exp(glast - gcs) | exp(glast)
-    float *dm;      // [H][64][64] decay mask
-    float *kb;      // [H][64][kd] K * beta
-    float *vb;      // [H][64][vd] V * beta
-    float *kbg;     // [H][64][kd] K * beta * exp(gcs)
-    float *qg;      // [H][64][kd] Q * exp(gcs)
-    float *kkd;     // [H][64][64] strictly lower (K_j . Kbeta_i) * decay
-    float *akq;     // [H][64][64] lower (K_j . Q_i) * decay
-    float *attn;    // [H][64][64] solved, unit diagonal
-    float *veff;    // [H][64][vd]
-    float *kcd;     // [H][64][kd]
+    float *qg;      // [64][128] Q * exp(gcs)
+    float *kcd;     // [64][128] attn @ K*beta*exp(gcs)
+    float *veff;    // [64][128] attn @ V*beta
+    float *kgt;     // [128][64] (K * exp(glast - gcs))^T
+    float *akq;     // [64][64] lower (K_j . Q_i) * decay
+    float *gl;      // exp(glast)
 };
 
 struct DnArgs {
@@ -56,6 +50,7 @@ struct DnArgs {
     int64_t n_tok;                       // tokens of the call
     int64_t g0;                          // first chunk of the group in flight
     int32_t H, kd, vd;
+    int32_t vec;                         // kd and vd are multiples of 4
 };
 
 // A scratch slot is one (chunk of the group, head): slot = c * H + h.
@@ -74,408 +69,550 @@ __device__ __forceinline__ DnChunk dn_chunk(const DnArgs &a, int slot) {
     return ck;
 }
 
-__device__ __forceinline__ const float *row_of(const float *base, const DnArgs &a, int64_t c0, int t, int h,
-                                               int dim) {
-    return base + ((c0 + t) * a.H + h) * (int64_t)dim;
+// Elements 4c .. 4c + 3 of row t of a chunk, dim a multiple of 4 (zeros past
+// the row or the chunk). Rows start on 4-byte boundaries.
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+
+__device__ __forceinline__ float4 dn_load4(const float *base, const DnArgs &a, const DnChunk &ck, int t, int c,
+                                           int dim) {
+    float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (t < ck.n && 4 * c < dim) {
+        const f4u x = *reinterpret_cast<const f4u *>(base + ((ck.c0 + t) * a.H + ck.h) * (int64_t)dim + 4 * c);
+        v = make_float4(x[0], x[1], x[2], x[3]);
+    }
+    return v;
 }
 
-// 1. grid (DN_PREP parts, slots): every part rebuilds the cumulative gate
-// of its slot (the g row staged in LDS by 64 lanes at once, then the serial
-// sum) and takes every DN_PREP-th slice of the elementwise work; part 0
-// writes the gate vectors.
-constexpr int DN_PREP = 8;
-
-__global__ __launch_bounds__(256) void k_dn_prep(DnArgs a, DnScratch s) {
-    const DnChunk ck = dn_chunk(a, blockIdx.y);
-    const int h = ck.h, part = blockIdx.x, n = ck.n, kd = a.kd, vd = a.vd;
-    __shared__ float gcs[DN_C], gex[DN_C];
-    float *gv = s.gv + (int64_t)ck.slot * (3 * DN_C + 1);
-    if (threadIdx.x < n) gcs[threadIdx.x] = a.g[(ck.c0 + threadIdx.x) * a.H + h];
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float run = 0.0f;
-        for (int t = 0; t < n; t++) {
-            run = __fadd_rn(run, gcs[t]);
-            gcs[t] = run;
-        }
-    }
-    __syncthreads();
-    const float glast = gcs[n - 1];
-    for (int t = threadIdx.x; t < n; t += 256) {
-        gex[t] = qk_expf(gcs[t]);
-        if (part == 0) {
-            gv[t] = gcs[t];
-            gv[DN_C + t] = gex[t];
-            gv[2 * DN_C + t] = qk_expf(__fsub_rn(glast, gcs[t]));
-        }
-    }
-    if (part == 0 && threadIdx.x == 0) gv[3 * DN_C] = qk_expf(glast);
-    __syncthreads();
-    const int first = part * 256 + threadIdx.x, stride = 256 * DN_PREP;
-    float *dm = s.dm + (int64_t)ck.slot * DN_C * DN_C;
-    for (int p = first; p < n * n; p += stride) {
-        const int i = p / n, j = p % n;
-        dm[i * DN_C + j] = i > j ? qk_expf(__fsub_rn(gcs[i], gcs[j])) : 0.0f;
-    }
-    const int64_t ho = (int64_t)ck.slot * DN_C;
-    // the rows in rounds of four elements per thread, every load of a
-    // round in flight before its products (64 x 128 elements: one round)
-    for (int p0 = first; p0 < n * kd; p0 += 4 * stride) {
-        float kv[4], qv[4], bv[4];
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int p = p0 + u * stride, t = p / kd, d = p % kd;
-            const bool in = p < n * kd;
-            kv[u] = in ? row_of(a.k, a, ck.c0, t, h, kd)[d] : 0.0f;
-            qv[u] = in ? row_of(a.q, a, ck.c0, t, h, kd)[d] : 0.0f;
-            bv[u] = in ? a.beta[(ck.c0 + t) * a.H + h] : 0.0f;
-        }
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int p = p0 + u * stride, t = p / kd, d = p % kd;
-            if (p < n * kd) {
-                const float kbv = __fmul_rn(kv[u], bv[u]);
-                const float ge = gex[t];
-                s.kb[(ho + t) * kd + d] = kbv;
-                s.kbg[(ho + t) * kd + d] = __fmul_rn(kbv, ge);
-                s.qg[(ho + t) * kd + d] = __fmul_rn(ge, qv[u]);
-            }
-        }
-    }
-    for (int p0 = first; p0 < n * vd; p0 += 4 * stride) {
-        float vv[4], bv[4];
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int p = p0 + u * stride, t = p / vd, e = p % vd;
-            const bool in = p < n * vd;
-            vv[u] = in ? row_of(a.v, a, ck.c0, t, h, vd)[e] : 0.0f;
-            bv[u] = in ? a.beta[(ck.c0 + t) * a.H + h] : 0.0f;
-        }
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int p = p0 + u * stride, t = p / vd, e = p % vd;
-            if (p < n * vd) s.vb[(ho + t) * vd + e] = __fmul_rn(vv[u], bv[u]);
-        }
-    }
+__device__ __forceinline__ float4 scale4(float4 v, float s) {
+    return make_float4(__fmul_rn(v.x, s), __fmul_rn(v.y, s), __fmul_rn(v.z, s), __fmul_rn(v.w, s));
 }
 
-// 2. grid (4 j-tiles, 4 i-tiles, slots); a 16x16 tile of (query i, key j) per
-// workgroup, the 16 K rows of its keys and the 16 Kbeta / Q rows of its
-// queries in LDS
-__global__ __launch_bounds__(256) void k_dn_dots(DnArgs a, DnScratch s) {
-    const DnChunk ck = dn_chunk(a, blockIdx.z);
-    const int h = ck.h, n = ck.n, kd = a.kd;
-    const int i0 = blockIdx.y * 16, j0 = blockIdx.x * 16;
-    if (i0 >= n || j0 >= n) return;                   // whole workgroup: tile outside the chunk
-    // tiles above the diagonal still run: they write the zeros the later
-    // phases read there (the reference's matrices hold 0.0f above it)
-    __shared__ float kj[16][DN_D + 1], kbi[16][DN_D + 1], qi[16][DN_D + 1];   // padded: row r on bank r
-    const int64_t ho = (int64_t)ck.slot * DN_C;
-    {
-        float vk[8], vb[8], vq[8];
-#pragma unroll
-        for (int u = 0; u < 8; u++) {                  // 8 * 256 = 16 rows of DN_D
-            const int p = u * 256 + threadIdx.x, r = p / DN_D, d = p % DN_D;
-            const bool jin = d < kd && j0 + r < n, iin = d < kd && i0 + r < n;
-            vk[u] = jin ? row_of(a.k, a, ck.c0, j0 + r, h, kd)[d] : 0.0f;
-            vb[u] = iin ? s.kb[(ho + i0 + r) * kd + d] : 0.0f;
-            vq[u] = iin ? row_of(a.q, a, ck.c0, i0 + r, h, kd)[d] : 0.0f;
-        }
-#pragma unroll
-        for (int u = 0; u < 8; u++) {
-            const int p = u * 256 + threadIdx.x, r = p / DN_D, d = p % DN_D;
-            kj[r][d] = vk[u];
-            kbi[r][d] = vb[u];
-            qi[r][d] = vq[u];
-        }
-    }
-    __syncthreads();
-    const int i = i0 + (threadIdx.x >> 4), j = j0 + (threadIdx.x & 15);
-    if (i >= n || j >= n) return;
-    const float *dm = s.dm + (int64_t)ck.slot * DN_C * DN_C;
-    float kk = 0.0f, kq = 0.0f;
-    if (i > j) {
-        float acc = 0.0f;
-        for (int d = 0; d < kd; d++) acc = __fadd_rn(acc, __fmul_rn(kj[threadIdx.x & 15][d], kbi[threadIdx.x >> 4][d]));
-        kk = __fmul_rn(acc, dm[i * DN_C + j]);
-    }
-    if (i >= j) {
-        float acc = 0.0f;
-        for (int d = 0; d < kd; d++) acc = __fadd_rn(acc, __fmul_rn(kj[threadIdx.x & 15][d], qi[threadIdx.x >> 4][d]));
-        kq = __fmul_rn(acc, i == j ? 1.0f : dm[i * DN_C + j]);
-    }
-    s.kkd[(ho + i) * DN_C + j] = kk;
-    s.akq[(ho + i) * DN_C + j] = kq;
+__device__ __forceinline__ bool finite(float x) { return fabsf(x) < __builtin_inff(); }
+__device__ __forceinline__ bool finite4(float4 v) { return finite(v.x) && finite(v.y) && finite(v.z) && finite(v.w); }
+
+__device__ __forceinline__ float dn_term(float acc, float c, float x) { return __fadd_rn(acc, __fmul_rn(c, x)); }
+
+// As the reference writes it where it skips a zero coefficient c.
+__device__ __forceinline__ float dn_term_skip(float acc, float c, float x) { return c != 0.0f ? dn_term(acc, c, x) : acc; }
+
+__device__ __forceinline__ float lane_value(float v, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
 
-// 3. one wave per slot, lane j solves column j of (I + L) X = -L, L the
-// strictly lower kkd (slm/chunked.c:196-213): X[i][j] = (-L[i][j] -
-// sum_{t<i} L[i][t] X[t][j]) / 1. The order is right-looking: as soon as
-// X[k][j] is known every later row adds its term k, so each row's sum
-// still runs t = 0, 1, 2, ... in the reference's order while the
-// dependent path is a few operations per row. The sums sit in registers
-// (both loops unrolled). LS[k] holds column k of L below the diagonal,
-// L[k+1 .. 63][k], from its first element, so row k's broadcast
-// coefficients arrive as a few aligned 16-byte reads issued together.
-// Dividing by the unit diagonal returns its operand unchanged (a quiet NaN
-// included), so the division is left out. Rows and columns past the chunk
-// run on stale scratch and are not stored; attn = X below the diagonal,
-// 1 on it, 0 above.
-__global__ __launch_bounds__(64) void k_dn_solve(DnArgs a, DnScratch s) {
-    const DnChunk ck = dn_chunk(a, blockIdx.x);
-    const int n = ck.n, j = threadIdx.x;
-    __shared__ float L[DN_C][DN_C + 1];                // lane j reads column j: no bank conflicts
-    __shared__ float4 LS[DN_C][DN_C / 4];              // LS[k][q] = L[k+1+4q .. k+4+4q][k]
-    const int64_t ho = (int64_t)ck.slot * DN_C;
-    {   // the whole 64x64 tile, sixteen 16-byte loads in flight per lane
-        const float4 *src = reinterpret_cast<const float4 *>(s.kkd + ho * DN_C);
-        float4 v[16];
+// ---- phase 1: everything of a chunk that the state does not enter ---------------
+// Grid (slots, 3 parts) of 512 threads; LDS leaves room for two workgroups
+// per CU:
+//   part 0  KK^T * decay, the solve, attn @ V*beta
+//   part 1  KK^T * decay, the solve, attn @ K*beta*exp(gcs)
+//   part 2  KQ^T * decay, Q*exp(gcs), (K*exp(glast - gcs))^T, exp(glast)
+// Parts 0 and 1 repeat the dots and the solve: it costs less than a second
+// launch with its loads. A workgroup is a chain of phases, each bound by
+// issue or latency (16 heads x 512 tokens, microseconds of one workgroup):
+// loads and the gates' sum 3.4, the dots 3.6 (4 rows from LDS for 4 chains),
+// the solve 4.3 (64 dependent steps), the apply 3.2. Against one launch per
+// phase, with the matrices through memory in between: 70 -> 22 us at 512
+// tokens, 38 -> 19 us at 100.
+constexpr int DN_WG = 512;
+
+// float4 column c of row t in the dots' operands: rows 2b of sixteen
+// consecutive b fall on sixteen different 16-byte columns.
+__device__ __forceinline__ int dn_swz(int t, int c) { return t * (DN_D / 4) + (c ^ ((t >> 1) & 15)); }
+
+// Element (i, j) of the triangular matrices: rows r, r + 8, ... of one column
+// lie 512 floats apart (two to an LDS read), rows 0 .. 7 on different banks.
+__device__ __forceinline__ int dn_tri(int i, int j) { return i * DN_C + (j ^ ((i & 7) << 3)); }
+
+// X = (I + L)^-1 - I below the diagonal (slm/chunked.c:196-213): X[i][j] =
+// (-L[i][j] - sum_{t<i} L[i][t] X[t][j]) / 1. Lane (j, rg) holds the sums of
+// rows rg, rg + 8, ... of column j; eight lanes side by side share a column.
+// Right-looking: as soon as X[k][j] is known every later row adds its term
+// k, so each row's sum runs t = 0, 1, 2, ... in the reference's order.
+// X[k][j] goes from its lane to the column's eight by DPP; column k + 2 of L
+// is read while step k runs. Dividing by the unit diagonal returns its
+// operand unchanged (a quiet NaN included), so the division is left out.
+// xs[m]: row rg + 8m (rows of a finished slot keep adding what is above the
+// diagonal of L, which nothing reads).
+__device__ __forceinline__ void dn_solve(const float *L, int j, int rg, float (&xs)[8]) {
+    float acc[8], nl[8], cf[3][8];
+    auto column = [&](int k) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < 16; u++) v[u] = src[u * 64 + j];
-        float *ls = &LS[0][0].x;
+        for (int m = 0; m < 8; m++)
+            if (m >= k / 8) cf[k % 3][m] = L[dn_tri(rg, k) + 8 * DN_C * m];
+    };
 #pragma unroll
-        for (int u = 0; u < 16; u++) {
-            const int p = (u * 64 + j) * 4, i = p / DN_C, t = p % DN_C;
-            const float e[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                L[i][t + c] = e[c];
-                if (i > t + c) ls[(t + c) * DN_C + (i - t - c - 1)] = e[c];
-            }
-        }
+    for (int m = 0; m < 8; m++) {
+        const int i = rg + 8 * m;
+        nl[m] = j < i ? -L[dn_tri(rg, j) + 8 * DN_C * m] : -0.0f;   // L is 0 from the diagonal on
+        acc[m] = xs[m] = 0.0f;
     }
-    __syncthreads();
-    float acc[DN_C], xs[DN_C];
-#pragma unroll
-    for (int i = 0; i < DN_C; i++) acc[i] = 0.0f;
+    column(0);
+    column(1);
 #pragma unroll
     for (int k = 0; k < DN_C; k++) {
-        const float x = __fsub_rn(-L[k][j], acc[k]);   // -L is -0 on and above the diagonal
-        xs[k] = x;
-        constexpr int nq_max = DN_C / 4;
-        const int nq = (DN_C - 1 - k + 3) / 4;          // compile-time after unrolling
-        float cf[DN_C];
-#pragma unroll
-        for (int q = 0; q < nq_max; q++) {
-            if (q < nq) {
-                const float4 c4 = LS[k][q];
-                cf[4 * q] = c4.x;
-                cf[4 * q + 1] = c4.y;
-                cf[4 * q + 2] = c4.z;
-                cf[4 * q + 3] = c4.w;
-            }
+        if (k + 2 < DN_C) column(k + 2);
+        asm volatile("" ::: "memory");                 // the reads stay two steps ahead
+        const int mk = k / 8, ok = k % 8;              // row k is slot mk of lane ok
+        const float x0 = __fsub_rn(nl[mk], acc[mk]);   // meant in lane ok
+        xs[mk] = rg == ok ? x0 : xs[mk];
+        int b = 0;                                     // its quad's copy, then the other quad's
+        switch (ok & 3) {
+            case 0: b = __builtin_amdgcn_mov_dpp(__float_as_int(x0), 0x00, 0xF, 0xF, true); break;
+            case 1: b = __builtin_amdgcn_mov_dpp(__float_as_int(x0), 0x55, 0xF, 0xF, true); break;
+            case 2: b = __builtin_amdgcn_mov_dpp(__float_as_int(x0), 0xAA, 0xF, 0xF, true); break;
+            default: b = __builtin_amdgcn_mov_dpp(__float_as_int(x0), 0xFF, 0xF, 0xF, true); break;
         }
+        const int o = dpp_hmirror(b);
+        const float x = __int_as_float((rg >> 2) == (ok >> 2) ? b : o);
+        float p[8];
 #pragma unroll
-        for (int i = k + 1; i < DN_C; i++) acc[i] = __fadd_rn(acc[i], __fmul_rn(cf[i - k - 1], x));
-        // keep one row's coefficients live at a time: the updates happen
-        // here, and the next row's reads stay below
+        for (int m = mk; m < 8; m++) p[m] = __fmul_rn(cf[k % 3][m], x);
 #pragma unroll
-        for (int i = k + 1; i < DN_C; i++) asm volatile("" : "+v"(acc[i]));
-        asm volatile("" ::: "memory");
-    }
-    if (j < n) {
-        float *attn = s.attn + ho * DN_C;
-#pragma unroll
-        for (int k = 0; k < DN_C; k++)
-            if (k < n) attn[k * DN_C + j] = j < k ? xs[k] : (j == k ? 1.0f : 0.0f);
+        for (int m = mk; m < 8; m++) acc[m] = __fadd_rn(acc[m], p[m]);
     }
 }
 
-// Phases 4, 6 and 7 read DN_B operands ahead of the dependent adds: every
-// scratch row index below stays under DN_C (rows past the chunk hold stale
-// data and meet a zero coefficient), and reads of the caller's arrays stop
-// at the chunk's last row.
-constexpr int DN_R = 4;                                // rows per lane in phase 4
-constexpr int DN_B = 8;                                // loads in flight per chain
-
-// 4. grid (8 row blocks, 2, slots), blocks past the chunk exit: a
-// workgroup computes eight rows of attn @ V*beta (y = 0) or
-// attn @ K*beta*exp(gcs) (y = 1). The rows of the right-hand matrix up to
-// the block's last row and the block's eight attn rows (j-major, so one
-// 16-byte read gives a lane its four rows' coefficients) are staged in LDS
-// with every load in flight at once; lane (row group, e) then runs four
-// rows' chains in the reference's j order from LDS. A zero coefficient
-// leaves a chain unchanged (the reference skips it). Columns j below the
-// group's first row belong to all four rows; the last few columns are
-// gated by j <= i. Rows past the chunk are computed and not stored.
-constexpr int DN_RB = 8;                               // rows per workgroup
-
-__global__ __launch_bounds__(256) void k_dn_apply(DnArgs a, DnScratch s) {
-    const DnChunk ck = dn_chunk(a, blockIdx.z);
-    const int n = ck.n, r0 = blockIdx.x * DN_RB;
-    if (r0 >= n) return;                               // whole workgroup: rows past the chunk
-    const int w = blockIdx.y ? a.kd : a.vd;
-    const int64_t ho = (int64_t)ck.slot * DN_C;
-    const float *src = blockIdx.y ? s.kbg + ho * a.kd : s.vb + ho * a.vd;
-    float *dst = blockIdx.y ? s.kcd + ho * a.kd : s.veff + ho * a.vd;
-    __shared__ float M[DN_C * DN_D];
-    __shared__ float4 Ct[DN_C][DN_RB / DN_R];          // Ct[j][g]: rows r0+4g .. r0+4g+3 at column j
-    const int rows = r0 + DN_RB < n ? r0 + DN_RB : n;  // right-hand rows 0 .. rows-1
-    const int total = rows * w;                        // <= 64 * 128 = 32 * 256
-    {
-        float v[32];
+// Rows wave + 8m of attn @ M (M [64][128] in LDS), two columns per lane. A
+// row of attn sits in one register (lane j: column j) and its elements
+// become wave-uniform factors by readlane. Row wave + 8m ends at column
+// wave + 8m; the columns from there to 8m + 7 are zeros. n8: 8-row slots
+// that hold rows of the chunk.
+__device__ __forceinline__ void dn_apply(const float (&at)[8], const float *M, int lane, int n8, float (&o)[8][2]) {
+    float x[4][2];
 #pragma unroll
-        for (int u = 0; u < 32; u++) {
-            const int p = u * 256 + threadIdx.x;
-            v[u] = p < total ? src[p] : 0.0f;
-        }
-        const float *arow = s.attn + (ho + r0) * DN_C;   // rows r0 .. r0+7 <= 63
-        const float c0 = arow[threadIdx.x], c1 = arow[256 + threadIdx.x];
+    for (int q = 0; q < 4; q++) x[q][0] = M[q * DN_D + lane], x[q][1] = M[q * DN_D + 64 + lane];
 #pragma unroll
-        for (int u = 0; u < 32; u++) {
-            const int p = u * 256 + threadIdx.x;
-            if (p < total) M[p] = v[u];
+    for (int mj = 0; mj < 8; mj++) {
+        if (mj >= n8) break;                           // uniform
+#pragma unroll
+        for (int h = 0; h < 2; h++) {                  // four columns of attn, the next four's rows in flight
+            float nx[4][2];
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int j = (8 * mj + 4 * h + 4 + q) & (DN_C - 1);
+                nx[q][0] = M[j * DN_D + lane];
+                nx[q][1] = M[j * DN_D + 64 + lane];
+            }
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int j = 8 * mj + 4 * h + q;
+                float c[8], p0[8], p1[8];
+#pragma unroll
+                for (int m = mj; m < 8; m++) c[m] = lane_value(at[m], j);
+#pragma unroll
+                for (int m = mj; m < 8; m++) {
+                    p0[m] = __fmul_rn(c[m], x[q][0]);
+                    p1[m] = __fmul_rn(c[m], x[q][1]);
+                }
+#pragma unroll
+                for (int m = mj; m < 8; m++) {
+                    o[m][0] = __fadd_rn(o[m][0], p0[m]);
+                    o[m][1] = __fadd_rn(o[m][1], p1[m]);
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < 4; q++) x[q][0] = nx[q][0], x[q][1] = nx[q][1];
         }
-        float *ct = &Ct[0][0].x;
-        ct[(threadIdx.x % DN_C) * DN_RB + threadIdx.x / DN_C] = c0;
-        ct[(threadIdx.x % DN_C) * DN_RB + 4 + threadIdx.x / DN_C] = c1;
+    }
+}
+
+// The same with the reference's skips, for a factor that is not finite.
+__device__ __forceinline__ void dn_apply_skip(const float (&at)[8], const float *M, int lane, float (&o)[8][2]) {
+#pragma unroll 1
+    for (int j = 0; j < DN_C; j++) {
+        const float x0 = M[j * DN_D + lane], x1 = M[j * DN_D + 64 + lane];
+#pragma unroll
+        for (int m = 0; m < 8; m++) {
+            const float c = lane_value(at[m], j);
+            o[m][0] = dn_term_skip(o[m][0], c, x0);
+            o[m][1] = dn_term_skip(o[m][1], c, x1);
+        }
+    }
+}
+
+__global__ __launch_bounds__(DN_WG) void k_dn_chunk(DnArgs a, DnScratch s) {
+    const DnChunk ck = dn_chunk(a, blockIdx.x);
+    const int part = blockIdx.y, n = ck.n, kd = a.kd;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    __shared__ float4 A[DN_C * DN_D / 4];              // K rows; then V*beta or K*beta*exp(gcs)
+    __shared__ float4 B[DN_C * DN_D / 4];              // K*beta or Q rows; then KK^T or KQ^T; then attn
+    __shared__ float gcs[DN_C], glast;                 // the gates' running sum; its last
+    __shared__ uint64_t etab[32];
+    __shared__ int bad;                                // a factor of the apply is not finite
+    // thread: float4 column c of rows t0, t0 + 16, ...
+    const int c = tid & 31, t0 = tid >> 5;
+    float4 kr[4], r2[4];                               // K; V (part 0) or Q (part 2)
+    const float *other = part == 0 ? a.v : a.q;
+    const int odim = part == 0 ? a.vd : kd;
+    if (a.vec) {                                       // uniform
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            kr[u] = dn_load4(a.k, a, ck, t0 + 16 * u, c, kd);
+            r2[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            if (part != 1) r2[u] = dn_load4(other, a, ck, t0 + 16 * u, c, odim);
+        }
+    } else {                                           // element by element through LDS
+        float *Af = reinterpret_cast<float *>(A), *Bf = reinterpret_cast<float *>(B);
+#pragma unroll 1
+        for (int p = tid; p < DN_C * DN_D; p += DN_WG) {
+            const int t = p / DN_D, d = p % DN_D;
+            const int64_t row = (ck.c0 + t) * a.H + ck.h;
+            Af[p] = t < n && d < kd ? a.k[row * kd + d] : 0.0f;
+            Bf[p] = part != 1 && t < n && d < odim ? other[row * odim + d] : 0.0f;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            kr[u] = A[(t0 + 16 * u) * (DN_D / 4) + c];
+            r2[u] = B[(t0 + 16 * u) * (DN_D / 4) + c];
+        }
+    }
+    float bt[4];                                       // beta of the thread's rows
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const int t = t0 + 16 * u;
+        bt[u] = t < n ? a.beta[(ck.c0 + t) * a.H + ck.h] : 0.0f;
+    }
+    if (wave == 0) {                                   // the gates' sums, lane t for token t
+        const float g = lane < n ? a.g[(ck.c0 + lane) * a.H + ck.h] : 0.0f;
+        if (lane < 32) etab[lane] = qk_exp2_32[lane];
+        if (lane == 0) bad = 0;
+        float run = 0.0f, mine = 0.0f;
+#pragma unroll 8
+        for (int t = 0; t < ((n + 7) & ~7); t++) {     // g past the chunk adds +0
+            run = __fadd_rn(run, lane_value(g, t));
+            mine = lane == t ? run : mine;
+        }
+        gcs[lane] = mine;
+        if (lane == 0) glast = run;
+    }
+    const int64_t ro = (int64_t)ck.slot * DN_C * DN_D; // a [64][128] (or [128][64]) array of the slot
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        const int t = t0 + 16 * u;
+        A[dn_swz(t, c)] = kr[u];
+        if (part == 2) {
+            B[dn_swz(t, c)] = r2[u];
+        } else {
+            kr[u] = scale4(kr[u], bt[u]);              // K * beta
+            B[dn_swz(t, c)] = kr[u];
+        }
     }
     __syncthreads();
-    const int rg = threadIdx.x / w, e = threadIdx.x % w;
-    const int i0 = r0 + rg * DN_R;
-    if (rg >= DN_RB / DN_R || i0 >= n) return;
-    const int last = i0 + DN_R - 1 < n - 1 ? i0 + DN_R - 1 : n - 1;
-    float acc[DN_R] = {0.0f, 0.0f, 0.0f, 0.0f};
-    auto term = [&](int j, const float4 c, float x, bool gate) __attribute__((always_inline)) {
-        const float cf[DN_R] = {c.x, c.y, c.z, c.w};
+    if (part == 2) {
+        // exp(gcs) * Q; (K * exp(glast - gcs))^T, 4 tokens a store
+        if (tid == 0) s.gl[ck.slot] = qk_expf_tab(glast, etab);
 #pragma unroll
-        for (int r = 0; r < DN_R; r++) {
-            const float k = (!gate || j <= i0 + r) ? cf[r] : 0.0f;
-            acc[r] = k != 0.0f ? __fadd_rn(acc[r], __fmul_rn(k, x)) : acc[r];
+        for (int u = 0; u < 4; u++) {                  // rows past the chunk are zeros
+            const int t = t0 + 16 * u;
+            const float4 qg = scale4(r2[u], qk_expf_tab(gcs[t], etab));
+            *reinterpret_cast<float4 *>(s.qg + ro + t * DN_D + 4 * c) = qg;
         }
-    };
-    int j0 = 0;
-    for (; j0 + DN_B <= i0; j0 += DN_B) {              // j < i0: a term of every row of the group
-        float xv[DN_B];
-        float4 c4[DN_B];
+        const float *Af = reinterpret_cast<const float *>(A);
+        const int tq = (tid & 15) * 4;
+        float gf[4];
 #pragma unroll
-        for (int u = 0; u < DN_B; u++) {
-            xv[u] = M[(j0 + u) * w + e];
-            c4[u] = Ct[j0 + u][rg];
+        for (int i = 0; i < 4; i++) gf[i] = qk_expf_tab(__fsub_rn(glast, gcs[tq + i]), etab);
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int d = (tid + DN_WG * u) >> 4;
+            float e[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int t = tq + i;
+                e[i] = t < n ? __fmul_rn(Af[4 * dn_swz(t, d >> 2) + (d & 3)], gf[i]) : 0.0f;
+            }
+            *reinterpret_cast<float4 *>(s.kgt + ro + d * DN_C + tq) = make_float4(e[0], e[1], e[2], e[3]);
         }
-#pragma unroll
-        for (int u = 0; u < DN_B; u++) term(j0 + u, c4[u], xv[u], false);
     }
-    for (int j = j0; j <= last; j++) term(j, Ct[j][rg], M[j * w + e], true);
+    // the dots, two rows against two per thread: the 496 tiles of row pairs
+    // below the diagonal, then 16 that hold the pairs (2b + 1, 2b)
+    float *D = reinterpret_cast<float *>(B);           // KK^T or KQ^T, once every thread is done with B
+    const int k4 = (kd + 3) / 4;
+    int i0, i1, j0, j1;
+    if (tid < 496) {                                   // p (p - 1) / 2 + q, q < p
+        int p = (int)((1.0f + __builtin_sqrtf(1.0f + 8.0f * (float)tid)) * 0.5f);
+        if (p * (p - 1) / 2 > tid) p--;
+        if (p * (p + 1) / 2 <= tid) p++;
+        i0 = 2 * p;
+        j0 = 2 * (tid - p * (p - 1) / 2);
+        i1 = i0 + 1;
+        j1 = j0 + 1;
+    } else {
+        j0 = 4 * (tid - 496);
+        i0 = j0 + 1;
+        j1 = j0 + 2;
+        i1 = j0 + 3;
+    }
+    float r[4] = {0.0f, 0.0f, 0.0f, 0.0f};             // (i0, j0), (i0, j1), (i1, j0), (i1, j1)
+    if (min(i0, i1) < n) {
+#pragma unroll 2
+        for (int d = 0; d < k4; d++) {
+            const float4 x0 = B[dn_swz(i0, d)], x1 = B[dn_swz(i1, d)];
+            const float4 y0 = A[dn_swz(j0, d)], y1 = A[dn_swz(j1, d)];
+            const float xa[4] = {x0.x, x0.y, x0.z, x0.w}, xb[4] = {x1.x, x1.y, x1.z, x1.w};
+            const float ya[4] = {y0.x, y0.y, y0.z, y0.w}, yb[4] = {y1.x, y1.y, y1.z, y1.w};
+            float p[4][4];
 #pragma unroll
-    for (int r = 0; r < DN_R; r++)
-        if (i0 + r <= last) dst[(i0 + r) * w + e] = acc[r];
+            for (int i = 0; i < 4; i++) {              // zeros past kd add +-0
+                p[0][i] = __fmul_rn(ya[i], xa[i]);
+                p[1][i] = __fmul_rn(yb[i], xa[i]);
+                p[2][i] = __fmul_rn(ya[i], xb[i]);
+                p[3][i] = __fmul_rn(yb[i], xb[i]);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) r[e] = __fadd_rn(r[e], p[e][i]);
+        }
+    }
+    float diag = 0.0f;                                 // part 2, wave 0: (lane, lane)
+    if (part == 2 && wave == 0) {
+#pragma unroll 2
+        for (int d = 0; d < k4; d++) {
+            const float4 x = B[dn_swz(lane, d)], y = A[dn_swz(lane, d)];
+            diag = dn_term(dn_term(dn_term(dn_term(diag, y.x, x.x), y.y, x.y), y.z, x.z), y.w, x.w);
+        }
+    }
+    const float gi[2] = {gcs[i0], gcs[i1]}, gj[2] = {gcs[j0], gcs[j1]};
+#pragma unroll
+    for (int e = 0; e < 4; e++)                        // the decay exp(gcs_i - gcs_j)
+        r[e] = __fmul_rn(r[e], qk_expf_tab(__fsub_rn(gi[e >> 1], gj[e & 1]), etab));
+    __syncthreads();                                   // every thread is done with A and B
+    if (i0 < n) {
+        D[dn_tri(i0, j0)] = r[0];
+        if (tid < 496) D[dn_tri(i0, j1)] = r[1];       // above the diagonal in the last tiles
+    }
+    if (i1 < n) {
+        if (tid < 496) D[dn_tri(i1, j0)] = r[2];       // another tile's in the last tiles
+        D[dn_tri(i1, j1)] = r[3];
+    }
+    if (part == 2) {
+        if (wave == 0) D[dn_tri(lane, lane)] = diag;   // the decay there is 1
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            const int e0 = (tid + DN_WG * u) * 4, i = e0 / DN_C, j = e0 % DN_C;
+            float e[4];
+#pragma unroll
+            for (int v = 0; v < 4; v++) e[v] = j + v <= i && i < n ? D[dn_tri(i, j + v)] : 0.0f;
+            *reinterpret_cast<float4 *>(s.akq + (int64_t)ck.slot * DN_C * DN_C + e0) =
+                make_float4(e[0], e[1], e[2], e[3]);
+        }
+        return;
+    }
+    // rows past the chunk: zeros, so that their solve and apply give zeros
+    for (int p = tid; p < (DN_C - n) * DN_C; p += DN_WG) D[dn_tri(n + p / DN_C, p % DN_C)] = 0.0f;
+    bool fin = true;
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        if (part == 0) r2[u] = scale4(r2[u], bt[u]);   // V * beta
+        else r2[u] = scale4(kr[u], qk_expf_tab(gcs[t0 + 16 * u], etab));   // K * beta * exp(gcs)
+        A[(t0 + 16 * u) * (DN_D / 4) + c] = r2[u];     // plain rows: the apply reads along a row
+        fin = fin && finite4(r2[u]);
+    }
+    if (!fin) bad = 1;
+    __syncthreads();
+    float xs[8];
+    const int j = tid >> 3, rg = tid & 7;
+    dn_solve(D, j, rg, xs);
+    __syncthreads();                                   // the solve is done with L
+#pragma unroll
+    for (int m = 0; m < 8; m++) {
+        const int i = rg + 8 * m;
+        D[dn_tri(i, j)] = j < i ? xs[m] : (j == i ? 1.0f : 0.0f);
+    }
+    __syncthreads();
+    float at[8], o[8][2];
+#pragma unroll
+    for (int m = 0; m < 8; m++) {
+        at[m] = D[dn_tri(wave + 8 * m, lane)];
+        o[m][0] = o[m][1] = 0.0f;
+    }
+    const float *M = reinterpret_cast<const float *>(A);
+    if (bad) dn_apply_skip(at, M, lane, o);
+    else dn_apply(at, M, lane, (n + 7) / 8, o);
+    float *dst = (part == 0 ? s.veff : s.kcd) + ro;
+#pragma unroll
+    for (int m = 0; m < 8; m++) {
+        dst[(wave + 8 * m) * DN_D + lane] = o[m][0];
+        dst[(wave + 8 * m) * DN_D + 64 + lane] = o[m][1];
+    }
 }
 
-// 5-7 for every chunk of the group in one launch. Each of the three is
-// local to a column e of the state: v_new[., e], the output column e and
-// the new state column e read only the state column e and per-chunk rows
-// every column shares. So a workgroup owns DN_E columns of one head, keeps
-// them in LDS and walks the group's chunks in order: grid
-// (ceil(vd / DN_E), H), no workgroup waits for another. A chunk's shared
-// rows (Q*exp(gcs), the decayed keys, K, the KQ^T decay rows and the gate
-// factors) go through registers into LDS, rows padded by one float so the
-// eight rows a wave reads sit in different banks; the next chunk's loads
-// are issued before this chunk's chains run. Each element's chains run
-// in the reference's order, as phases 5-7 above do.
+// ---- phase 2: the carried state ----------------------------------------------------
+// A workgroup owns DN_E columns of one head's state, keeps them in LDS and
+// walks the group's chunks in order; v_new[., e], the output column e and
+// the new state column e read only the state column e and rows that every
+// column shares, so no workgroup waits for another. Lane (t, e) runs the two
+// chains over the state (query and decayed key of token t), then, over
+// v_new, the output chain of (t, e) and the state chains of (t, e) and
+// (t + 64, e). The four lanes of a quad have one t: each loads a quarter of
+// that row's coefficients straight from the scratch (16-byte loads, issued
+// while the other half of a chunk computes) and gets the rest by a quad
+// broadcast inside the multiply, so LDS carries only the state and v_new.
+// That multiply takes 4 cycles a wave against 2, but reading every
+// coefficient from LDS would bind earlier (3 reads per 2 terms). Measured:
+// 2.9 ns a SIMD for a product and its sum in a loop of these alone, 3.9 ns
+// here with the barriers and the reads; the products on the matrix cores (an
+// fp32 MFMA of one term rounds a product as the multiply does) took 3.2 ns.
+// With the coefficients staged in LDS, one output per lane and the skips in
+// the loop, 16 heads x 512 tokens took 91 us; 43 us here.
 constexpr int DN_E = 8;                                // state columns per workgroup
-constexpr int DN_RS = DN_D + 1;                        // padded LDS row of DN_D floats
-constexpr int DN_CS = DN_C + 1;                        // padded LDS row of DN_C floats
+constexpr int DN_SS = DN_D + 4;                        // LDS row of a state column
+constexpr int DN_VS = DN_C + 4;                        // LDS row of a v_new column
 
-// Lane (t, e) runs both chains of phase 5 and, over one loop, the output
-// chain of (t, e) and the state chains of (t, e) and (t + 64, e).
-__global__ __launch_bounds__(512) void k_dn_carry(DnArgs a, DnScratch s, int gc) {
-    constexpr int PR = DN_C * DN_D / 512, PA = DN_C * DN_C / 512;   // row / KQ^T elements per lane
-    __shared__ float Qs[DN_C * DN_RS], Ks[DN_C * DN_RS], Kr[DN_C * DN_RS], As[DN_C * DN_CS];
-    __shared__ float S[DN_D][DN_E], vn[DN_C][DN_E], gf[DN_C + 1];
-    const int h = blockIdx.y, e0 = blockIdx.x * DN_E, kd = a.kd, vd = a.vd;
-    const int tid = threadIdx.x, el = tid % DN_E, e = e0 + el, t = tid / DN_E;
+// v of lane Q of the quad.
+template <int Q>
+__device__ __forceinline__ float quad(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), Q * 0x55, 0xF, 0xF, true));
+}
+
+// The products of four terms of N chains (coefficients from quad lane Q,
+// factors x), each beside the sum that takes the product of four terms
+// before (p): a chain's next sum comes 2N instructions after its last, and
+// every product has a register of its own, so neither waits. The empty asm
+// keeps that order.
+template <int Q, int N>
+__device__ __forceinline__ void quad_terms(float (&acc)[N], float (&p)[4][N], const float4 (&cf)[N], float4 x,
+                                           bool first) {
+    const float xe[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const float ce = e == 0 ? cf[i].x : e == 1 ? cf[i].y : e == 2 ? cf[i].z : cf[i].w;
+            float m = __fmul_rn(quad<Q>(ce), xe[e]);
+            if (!first) acc[i] = __fadd_rn(acc[i], p[e][i]);
+            asm volatile("" : "+v"(m), "+v"(acc[i]));
+            p[e][i] = m;
+        }
+}
+
+// The chains over blocks of 16 elements of a column at col (LDS), a block's
+// elements read while the one before it computes.
+template <int N, int NB>
+__device__ __forceinline__ void dn_chains(float (&acc)[N], const float4 (&cf)[NB][N], const float *col, int nb) {
+    const float4 *x = reinterpret_cast<const float4 *>(col);
+    float4 cur[4], nxt[4];
+    float p[4][N];
+#pragma unroll
+    for (int i = 0; i < 4; i++) cur[i] = x[i];
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+        if (b + 1 < NB)
+#pragma unroll
+            for (int i = 0; i < 4; i++) nxt[i] = x[4 * (b + 1) + i];
+        asm volatile("" ::: "memory");                 // the reads stay above this block's terms
+        quad_terms<0>(acc, p, cf[b], cur[0], b == 0);
+        quad_terms<1>(acc, p, cf[b], cur[1], false);
+        quad_terms<2>(acc, p, cf[b], cur[2], false);
+        quad_terms<3>(acc, p, cf[b], cur[3], false);
+        if (b + 1 >= nb) break;                        // uniform
+#pragma unroll
+        for (int i = 0; i < 4; i++) cur[i] = nxt[i];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+#pragma unroll
+        for (int i = 0; i < N; i++) acc[i] = __fadd_rn(acc[i], p[e][i]);
+}
+
+__global__ __launch_bounds__(512) void k_dn_carry(DnArgs a, DnScratch s, int gc, int ncol) {
+    __shared__ __align__(16) float S[DN_E * DN_SS], V[DN_E * DN_VS];
+    __shared__ int bad;                                // the state holds or held an inf or NaN
+    // workgroups of one head on one XCD where the heads allow it: they
+    // read the same rows
+    int h, cg;
+    if ((a.H & 7) == 0) {
+        const int x = blockIdx.x >> 3;
+        h = (blockIdx.x & 7) + 8 * (x / ncol);
+        cg = x % ncol;
+    } else {
+        h = blockIdx.x / ncol;
+        cg = blockIdx.x % ncol;
+    }
+    const int e0 = cg * DN_E, kd = a.kd, vd = a.vd;
+    const int tid = threadIdx.x, el = tid % DN_E, e = e0 + el, t = tid / DN_E, ql = tid & 3;
     const bool col = e < vd;
     float *st = a.state + (int64_t)h * kd * vd;
+    if (tid == 0) bad = 0;
+    __syncthreads();
     for (int p = tid; p < DN_D * DN_E; p += 512) {
-        const int d = p / DN_E, c = p % DN_E;
-        S[d][c] = d < kd && e0 + c < vd ? st[(int64_t)d * vd + e0 + c] : 0.0f;
+        const int d = p / DN_E, cc = p % DN_E;
+        const float x = d < kd && e0 + cc < vd ? st[(int64_t)d * vd + e0 + cc] : 0.0f;
+        S[cc * DN_SS + d] = x;
+        if (!finite(x)) bad = 1;
     }
+    constexpr int B5 = DN_D / 16, B6 = DN_C / 16;
+    float4 c5[B5][2], c6[B6][3];
+    float ve, gl;
+    auto load5 = [&](int c) __attribute__((always_inline)) {
+        const int64_t ro = (int64_t)(c * a.H + h) * DN_C * DN_D + t * DN_D;
+#pragma unroll
+        for (int b = 0; b < B5; b++) {
+            c5[b][0] = *reinterpret_cast<const float4 *>(s.qg + ro + 16 * b + 4 * ql);
+            c5[b][1] = *reinterpret_cast<const float4 *>(s.kcd + ro + 16 * b + 4 * ql);
+        }
+        ve = s.veff[ro + (col ? e : 0)];
+    };
+    auto load6 = [&](int c) __attribute__((always_inline)) {
+        const int64_t slot = c * a.H + h;
+        const float *aq = s.akq + slot * DN_C * DN_C + t * DN_C, *kg = s.kgt + slot * DN_C * DN_D + t * DN_C;
+#pragma unroll
+        for (int b = 0; b < B6; b++) {
+            c6[b][0] = *reinterpret_cast<const float4 *>(aq + 16 * b + 4 * ql);
+            c6[b][1] = *reinterpret_cast<const float4 *>(kg + 16 * b + 4 * ql);
+            c6[b][2] = *reinterpret_cast<const float4 *>(kg + 64 * DN_C + 16 * b + 4 * ql);
+        }
+        gl = s.gl[slot];
+    };
+    load5(0);
+    load6(0);
+    __syncthreads();
+    const int nd = (kd + 15) / 16;
     for (int c = 0; c < gc; c++) {
         const DnChunk ck = dn_chunk(a, c * a.H + h);
         const int n = ck.n;
-        const int64_t ho = (int64_t)ck.slot * DN_C;
-        // the chunk's shared rows: every load in flight, then into LDS
-        float rq[PR], rc[PR], rk[PR], ra[PA], rg;
-#pragma unroll
-        for (int u = 0; u < PR; u++) {
-            const int p = tid + 512 * u, tt = p / kd, d = p - tt * kd;
-            const bool in = tt < n;
-            rq[u] = in ? s.qg[(ho + tt) * kd + d] : 0.0f;
-            rc[u] = in ? s.kcd[(ho + tt) * kd + d] : 0.0f;
-            rk[u] = in ? row_of(a.k, a, ck.c0, tt, h, kd)[d] : 0.0f;
-        }
-#pragma unroll
-        for (int u = 0; u < PA; u++) {
-            const int p = tid + 512 * u;
-            ra[u] = p / DN_C < n ? s.akq[ho * DN_C + p] : 0.0f;
-        }
-        // exp(glast - gcs[t]) for t < 64, exp(glast) at 64
-        rg = tid <= DN_C ? s.gv[(int64_t)ck.slot * (3 * DN_C + 1) + 2 * DN_C + tid] : 0.0f;
-        __syncthreads();                               // the previous chunk's reads of the rows done
-#pragma unroll
-        for (int u = 0; u < PR; u++) {
-            const int p = tid + 512 * u, tt = p / kd, d = p - tt * kd;
-            if (tt < DN_C) {
-                Qs[tt * DN_RS + d] = rq[u];
-                Ks[tt * DN_RS + d] = rc[u];
-                Kr[tt * DN_RS + d] = rk[u];
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < PA; u++) {
-            const int p = tid + 512 * u;
-            As[(p / DN_C) * DN_CS + p % DN_C] = ra[u];
-        }
-        if (tid <= DN_C) gf[tid] = rg;
-        __syncthreads();
-        // 5: the chains against the state (Q*exp(gcs) and the decayed
-        // keys, skipping zero coefficients as the reference does); v_new
-        float ai = 0.0f;
-        if (t < n && col) {
-            float vp = 0.0f;
-            const float *qr = Qs + t * DN_RS, *kr = Ks + t * DN_RS;
-#pragma unroll 8
+        // the chains against the state: query and decayed key of token t
+        float a5[2] = {0.0f, 0.0f};
+        if (bad) {                                     // uniform; with the reference's skips
+            const float *qg = s.qg + (int64_t)ck.slot * DN_C * DN_D + t * DN_D;
+            const float *kc = s.kcd + (int64_t)ck.slot * DN_C * DN_D + t * DN_D;
+#pragma unroll 1
             for (int d = 0; d < kd; d++) {
-                const float x = S[d][el], qv = qr[d], kv = kr[d];
-                ai = qv != 0.0f ? __fadd_rn(ai, __fmul_rn(qv, x)) : ai;
-                vp = kv != 0.0f ? __fadd_rn(vp, __fmul_rn(kv, x)) : vp;
+                const float x = S[el * DN_SS + d];
+                a5[0] = dn_term_skip(a5[0], qg[d], x);
+                a5[1] = dn_term_skip(a5[1], kc[d], x);
             }
-            vn[t][el] = __fsub_rn(s.veff[(ho + t) * vd + e], vp);
+        } else {
+            dn_chains(a5, c5, S + el * DN_SS, nd);
         }
+        V[el * DN_VS + t] = t < n && col ? __fsub_rn(ve, a5[1]) : 0.0f;
         __syncthreads();
-        // 6 and 7 over u: the output row's chain (the intra-chunk attention
-        // on v_new) and the state's for d = t and t + 64, with
-        // K * exp(glast - gcs) rounded as the reference forms it
-        const float *kq = As + t * DN_CS;
-        const int d0 = t, d1 = t + 64;
-        float acc6 = 0.0f, acc0 = 0.0f, acc1 = 0.0f;
-#pragma unroll 4
-        for (int u = 0; u < n; u++) {
-            const float x = vn[u][el], g = gf[u];
-            acc6 = __fadd_rn(acc6, __fmul_rn(kq[u], x));
-            acc0 = __fadd_rn(acc0, __fmul_rn(__fmul_rn(Kr[u * DN_RS + d0], g), x));
-            acc1 = __fadd_rn(acc1, __fmul_rn(__fmul_rn(Kr[u * DN_RS + d1], g), x));
-        }
-        if (col) {
-            if (t < n) a.out[((ck.c0 + t) * a.H + h) * (int64_t)vd + e] = __fadd_rn(ai, acc6);
-            if (d0 < kd) S[d0][el] = __fadd_rn(__fmul_rn(S[d0][el], gf[DN_C]), acc0);
-            if (d1 < kd) S[d1][el] = __fadd_rn(__fmul_rn(S[d1][el], gf[DN_C]), acc1);
-        }
+        if (c + 1 < gc) load5(c + 1);
+        // over v_new: the intra-chunk attention row t, the state rows t, t + 64
+        float a6[3] = {0.0f, 0.0f, 0.0f};
+        dn_chains(a6, c6, V + el * DN_VS, (n + 15) / 16);
+        if (t < n && col) a.out[((ck.c0 + t) * a.H + h) * (int64_t)vd + e] = __fadd_rn(a5[0], a6[0]);
+        float *s0 = &S[el * DN_SS + t];
+        const float n0 = t < kd ? __fadd_rn(__fmul_rn(s0[0], gl), a6[1]) : 0.0f;
+        const float n1 = t + 64 < kd ? __fadd_rn(__fmul_rn(s0[64], gl), a6[2]) : 0.0f;
+        s0[0] = n0;
+        s0[64] = n1;
+        if (!finite(n0) || !finite(n1)) bad = 1;
+        if (c + 1 < gc) load6(c + 1);
+        __syncthreads();
     }
-    __syncthreads();
     for (int p = tid; p < DN_D * DN_E; p += 512) {
-        const int d = p / DN_E, c = p % DN_E;
-        if (d < kd && e0 + c < vd) st[(int64_t)d * vd + e0 + c] = S[d][c];
+        const int d = p / DN_E, cc = p % DN_E;
+        if (d < kd && e0 + cc < vd) st[(int64_t)d * vd + e0 + cc] = S[cc * DN_SS + d];
     }
 }
 
 // ---- launcher -----------------------------------------------------------------
-// Phases 1-4 read only their chunk's own inputs, so they run for a group
-// of chunks at once (one launch per phase over every (chunk, head) slot of
-// the group); phases 5-7 carry the state and run chunk after chunk. A
-// group holds at most DN_SLOTS slots (one head's slot is about 263 KB of
-// scratch at head dims 128), and at least one chunk.
+// The chunks go in groups of at most DN_SLOTS (chunk, head) slots (147 KB of
+// scratch each) and at least one chunk.
 constexpr int DN_SLOTS = 256;
 
 static int dn_group(int32_t H, int64_t n_tok) {
@@ -485,10 +622,9 @@ static int dn_group(int32_t H, int64_t n_tok) {
 }
 
 size_t deltanet_scratch_bytes(int32_t H, int32_t kd, int32_t vd, int64_t n_tok) {
+    (void)kd, (void)vd;                                // rows are padded to DN_D
     const size_t slots = (size_t)dn_group(H, n_tok) * (size_t)H;
-    const size_t per = (size_t)(3 * DN_C + 1) + 4 * (size_t)DN_C * DN_C + 4 * (size_t)DN_C * kd +
-                       2 * (size_t)DN_C * vd;
-    return (per * slots + 11 * 64) * sizeof(float) + 256;   // 11 arrays, each rounded up to 64 floats
+    return (slots * (4 * DN_C * DN_D + DN_C * DN_C + 1) + 6 * 64) * sizeof(float) + 256;
 }
 
 hipError_t launch_deltanet(const float *q, const float *k, const float *v, const float *g, const float *beta,
@@ -497,34 +633,27 @@ hipError_t launch_deltanet(const float *q, const float *k, const float *v, const
     if (kd > DN_D || vd > DN_D || n_tok < 1 || H < 1) return hipErrorInvalidValue;
     const int G = dn_group(H, n_tok);
     const size_t slots = (size_t)G * (size_t)H;
-    float *p = static_cast<float *>(scratch);
+    float *p = reinterpret_cast<float *>((reinterpret_cast<uintptr_t>(scratch) + 255) & ~(uintptr_t)255);
     auto take = [&](size_t n_floats) {
         float *r = p;
         p += (n_floats + 63) & ~(size_t)63;            // 256-byte aligned arrays
         return r;
     };
     DnScratch s;
-    s.gv = take(slots * (3 * DN_C + 1));
-    s.dm = take(slots * DN_C * DN_C);
-    s.kkd = take(slots * DN_C * DN_C);
+    s.qg = take(slots * DN_C * DN_D);
+    s.kcd = take(slots * DN_C * DN_D);
+    s.veff = take(slots * DN_C * DN_D);
+    s.kgt = take(slots * DN_C * DN_D);
     s.akq = take(slots * DN_C * DN_C);
-    s.attn = take(slots * DN_C * DN_C);
-    s.kb = take(slots * DN_C * kd);
-    s.kbg = take(slots * DN_C * kd);
-    s.qg = take(slots * DN_C * kd);
-    s.kcd = take(slots * DN_C * kd);
-    s.vb = take(slots * DN_C * vd);
-    s.veff = take(slots * DN_C * vd);
+    s.gl = take(slots);
+    const int vec = kd % 4 == 0 && vd % 4 == 0;
     const int64_t chunks = (n_tok + DN_C - 1) / DN_C;
+    const int ncol = (vd + DN_E - 1) / DN_E;
     for (int64_t g0 = 0; g0 < chunks; g0 += G) {
         const int gc = (int)(chunks - g0 < G ? chunks - g0 : G);   // chunks in this group
-        const unsigned gs = (unsigned)(gc * H);                     // slots in this group
-        DnArgs a{q, k, v, g, beta, state, out, n_tok, g0, H, kd, vd};
-        hipLaunchKernelGGL(k_dn_prep, dim3(DN_PREP, gs), dim3(256), 0, st, a, s);
-        hipLaunchKernelGGL(k_dn_dots, dim3(4, 4, gs), dim3(256), 0, st, a, s);
-        hipLaunchKernelGGL(k_dn_solve, dim3(gs), dim3(64), 0, st, a, s);
-        hipLaunchKernelGGL(k_dn_apply, dim3(DN_C / DN_RB, 2, gs), dim3(256), 0, st, a, s);
-        hipLaunchKernelGGL(k_dn_carry, dim3((vd + DN_E - 1) / DN_E, H), dim3(512), 0, st, a, s, gc);
+        DnArgs a{q, k, v, g, beta, state, out, n_tok, g0, H, kd, vd, vec};
+        hipLaunchKernelGGL(k_dn_chunk, dim3((unsigned)(gc * H), 3), dim3(DN_WG), 0, st, a, s);
+        hipLaunchKernelGGL(k_dn_carry, dim3((unsigned)(ncol * H)), dim3(512), 0, st, a, s, gc, ncol);
     }
     return hipGetLastError();
 }

@@ -55,7 +55,8 @@ QK_EXPF_DATA uint64_t qk_exp2_32[32] = {
 QK_EXPF_FN uint64_t qk_bits64(double d) { uint64_t u; memcpy(&u, &d, 8); return u; }
 QK_EXPF_FN double qk_double(uint64_t u) { double d; memcpy(&d, &u, 8); return d; }
 
-QK_EXPF_FN float qk_expf(float x) {
+/* tab: a copy of qk_exp2_32 (a kernel with many calls keeps one in LDS). */
+QK_EXPF_FN float qk_expf_tab(float x, const uint64_t *tab) {
     /* Beyond these the result is +inf / +0 (glibc's own cut-offs: the
        largest x whose exp rounds to a finite float, and the point below
        which it rounds to zero). NaN propagates quietened, as x + x. */
@@ -74,13 +75,15 @@ QK_EXPF_FN float qk_expf(float x) {
     const uint64_t ki = qk_bits64(kb);
     const double kd = kb - round_shift;
     const double r = __builtin_fma(inv_ln2_n, xd, -kd);
-    const double scale = qk_double(qk_exp2_32[ki & 31] + (ki << 47));
+    const double scale = qk_double(tab[ki & 31] + (ki << 47));
     const double hi = __builtin_fma(c3, r, c2);
     const double r2 = r * r;
     double p = __builtin_fma(c1, r, 1.0);
     p = __builtin_fma(hi, r2, p);
     return (float)(p * scale);
 }
+
+QK_EXPF_FN float qk_expf(float x) { return qk_expf_tab(x, qk_exp2_32); }
 
 #undef QK_EXPF_FN
 #undef QK_EXPF_DATA

@@ -112,6 +112,31 @@ def test_deltanet_ragged_head_dims(lib, orc):
     assert_bits_equal(host(dst), want_s, "state")
 
 
+@pytest.mark.parametrize("H,kd,vd,n_tok", [(1, 1, 1, 1), (8, 7, 127, 65), (3, 127, 3, 63), (2, 100, 128, 129),
+                                           (24, 96, 64, 70), (8, 128, 120, 2)])
+@pytest.mark.parametrize("special", ["", "v", "k", "state"])
+def test_deltanet_splits(lib, orc, H, kd, vd, n_tok, special):
+    """The edges of the kernels' splits: head dims that the wide loads and
+    the 16-element blocks do not divide, heads with and without the XCD
+    order, chunks of one token and one past a chunk; and the factors whose
+    zero coefficients the reference skips, infinite or NaN."""
+    step(f"deltanet splits H={H} kd={kd} vd={vd} n={n_tok} special={special}")
+    q, k, v, g, b = ssm_inputs(n_tok, H=H, kd=kd, vd=vd, seed=H * kd + n_tok, zero_rows=n_tok > 3)
+    st = state0(H, kd, vd, kd)
+    bad = {"v": v, "k": k, "state": st}.get(special)
+    if bad is not None:
+        flat = bad.reshape(-1)
+        flat[flat.size // 3] = np.inf
+        flat[flat.size // 2] = np.nan
+        flat[0] = -np.inf
+    with np.errstate(all="ignore"):
+        want_o, want_s = orc.deltanet_chunked(q, k, v, g, b, st)
+    dst = dev(st)
+    out = lib.deltanet_chunked(dev(q), dev(k), dev(v), dev(g), dev(b), dst)
+    assert_bits_equal(host(out), want_o, "out")
+    assert_bits_equal(host(dst), want_s, "state")
+
+
 def test_deltanet_host_seam(lib, orc):
     """The body the seam gives chunked_ssm_step_f32: host buffers, one head."""
     step("deltanet host seam")
