@@ -278,11 +278,12 @@ __global__ __launch_bounds__(DN_WG) void k_dn_chunk(DnArgs a, DnScratch s) {
         if (lane < 32) etab[lane] = qk_exp2_32[lane];
         if (lane == 0) bad = 0;
         float run = 0.0f, mine = 0.0f;
-#pragma unroll 8
-        for (int t = 0; t < ((n + 7) & ~7); t++) {     // g past the chunk adds +0
-            run = __fadd_rn(run, lane_value(g, t));
-            mine = lane == t ? run : mine;
-        }
+        for (int t = 0; t < n; t += 8)                 // g past the chunk adds +0
+#pragma unroll
+            for (int q = 0; q < 8; q++) {
+                run = __fadd_rn(run, lane_value(g, t + q));
+                mine = lane == t + q ? run : mine;
+            }
         gcs[lane] = mine;
         if (lane == 0) glast = run;
     }

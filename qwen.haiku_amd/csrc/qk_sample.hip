@@ -21,8 +21,8 @@
 //    k, plus the block's own earlier candidates). Those with a count
 //    below k are the entering events, listed in index order with their
 //    values (k_smp_events);
-//  * the final slots: in closed form when the values are distinct, else
-//    one wave replays the events in order on the k slots; then the rest
+//  * the final slots: in closed form (past SMP_NMAX elements one wave
+//    replays the events in order on the k slots); then the rest
 //    of the chain on the k survivors as the reference writes it
 //    (k_smp_pick).
 // A NaN logit after the first k never enters and never compares >=, so it
@@ -278,6 +278,17 @@ constexpr int SMP_LIST_MAX = 16384;                    // keys of the prefix lis
 constexpr int SMP_WG = 1024;                           // threads of the selection kernels (16 waves)
 constexpr int SMP_SBMAX = 4096;                        // largest block
 
+// Blocks of sb logits, the first of them cut into blocks of 1024: in the
+// first logits most still enter, and a block's events are found by one
+// workgroup. per = sb / 1024.
+__host__ __device__ __forceinline__ int64_t smp_base(int32_t b, int32_t per) {
+    return b < per ? (int64_t)b * SMP_BLOCK : (int64_t)(b - per + 1) * per * SMP_BLOCK;
+}
+static int32_t smp_blocks_of(int64_t n, int32_t per) {
+    const int64_t sb = (int64_t)per * SMP_BLOCK;
+    return (int32_t)(n <= sb ? (n + SMP_BLOCK - 1) / SMP_BLOCK : per + (n - 1) / sb);
+}
+
 __device__ __forceinline__ float smp_load(const float *logits, int64_t n, int64_t i, int32_t k, int32_t &nan_fill) {
     if (i >= n) return -__builtin_inff();
     const float x = logits[i];
@@ -396,12 +407,9 @@ __host__ __device__ constexpr int smp_regs(int32_t k) { return k <= 64 ? 1 : (k 
 // initial fill holds a NaN. Each wave sorts its 64 * PER keys in
 // registers, then a tree of merges leaves the block's top 64R in wave 0.
 template <int PER, int R>
-__global__ __launch_bounds__(SMP_WG) void k_smp_blocks(float *logits, int64_t n, int32_t k, float *tops,
-                                                       int32_t *nan_flag, SmpPen pp) {
-    __shared__ uint32_t lds[16 * 64 * R];
-    __shared__ float xs[PER * SMP_WG];
+__device__ __forceinline__ void blocks_body(float *logits, int64_t n, int32_t k, float *tops, int32_t *nan_flag,
+                                            const SmpPen &pp, int64_t b0, uint32_t *lds, float *xs) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int64_t b0 = (int64_t)blockIdx.x * (PER * SMP_WG);
     const int64_t base = b0 + wave * 64 * PER;
     float xv[PER];
 #pragma unroll
@@ -445,6 +453,16 @@ __global__ __launch_bounds__(SMP_WG) void k_smp_blocks(float *logits, int64_t n,
     }
 }
 
+template <int PER, int R>
+__global__ __launch_bounds__(SMP_WG) void k_smp_blocks(float *logits, int64_t n, int32_t k, float *tops,
+                                                       int32_t *nan_flag, SmpPen pp) {
+    __shared__ uint32_t lds[16 * 64 * R];
+    __shared__ float xs[PER * SMP_WG];
+    const int64_t b0 = smp_base(blockIdx.x, PER);
+    if (PER > 1 && blockIdx.x < PER) blocks_body<1, R>(logits, n, k, tops, nan_flag, pp, b0, lds, xs);
+    else blocks_body<PER, R>(logits, n, k, tops, nan_flag, pp, b0, lds, xs);
+}
+
 // Block b's entering events. With P = the logits before the block and
 // T = the k-th largest of P, a logit of the block can enter only if it
 // exceeds T (in block 0, anything above -inf); such a logit v enters iff
@@ -461,7 +479,11 @@ __global__ __launch_bounds__(SMP_WG) void k_smp_blocks(float *logits, int64_t n,
 // waves' tops (Hillis-Steele over 16 waves) and the wave's own earlier
 // sub-chunks. A candidate's count is then a binary search in that sorted
 // top plus the earlier lanes of its sub-chunk, read lane by lane. A block
-// with at most 64 candidates skips the scan: one wave holds them all.
+// with at most 64 candidates skips the scan: one wave holds them all. Up to
+// 512 the workgroup compares each with those before it, two or four threads
+// a candidate; the scan is left to the first blocks. At top-k 256 and 248320
+// logits it took 24 us in each of the first five blocks of 4096, and the
+// kernel with it 30 us; now 13 us, the last blocks' merges.
 template <int R>
 __device__ __forceinline__ void wave_put(uint32_t *dst, const uint32_t (&v)[R]) {
     const int lane = threadIdx.x & 63;
@@ -475,22 +497,28 @@ __device__ __forceinline__ void wave_get(uint32_t (&v)[R], const uint32_t *src) 
     for (int r = 0; r < R; r++) v[r] = src[64 * r + lane];
 }
 
+constexpr int SMP_CAND = 512;                          // candidates compared pair by pair
+
+template <int R>
+struct EvLds {
+    uint32_t lds[16 * 64 * R];                         // merge exchanges, then each wave's running top
+    uint32_t pb[64 * R];                               // the top of P, sorted
+    int32_t ecnt[64];                                  // candidates, then events per sub-chunk; offsets
+    __align__(16) uint32_t ck[SMP_CAND];               // few candidates: keys, indices, values
+    int32_t ci[SMP_CAND];
+    float cv[SMP_CAND];
+    int32_t ncand;
+};
+
 template <int PER, int R>
-__global__ __launch_bounds__(SMP_WG) void k_smp_events(const float *logits, int64_t n, int32_t k,
-                                                       const float *tops, int32_t *ev_idx, float *ev_val,
-                                                       int32_t *ev_n) {
-    constexpr int SB = PER * SMP_WG;
+__device__ __forceinline__ void events_body(const float *logits, int64_t n, int32_t k, const float *tops,
+                                            int32_t *ev_idx, float *ev_val, int32_t *ev_n, int64_t base,
+                                            EvLds<R> &sh) {
     constexpr int LB = 16 / R;                         // lists loaded per batch (a power of two)
-    __shared__ uint32_t lds[16 * 64 * R];              // merge exchanges, then each wave's running top
-    __shared__ uint32_t pb[64 * R];                    // the top of P, sorted
-    __shared__ int32_t ecnt[16 * PER];                 // candidates, then events per sub-chunk; offsets
-    __shared__ uint32_t c1k[64];                       // at most 64 candidates: keys, indices, values
-    __shared__ int32_t c1i[64];
-    __shared__ float c1v[64];
-    __shared__ int32_t ncand_sh;
+    uint32_t *lds = sh.lds, *pb = sh.pb;
+    int32_t *ecnt = sh.ecnt;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int32_t b = blockIdx.x;
-    const int64_t base = (int64_t)b * SB;
     // the block's logits first, so their loads overlap the merges
     int32_t nan_fill = 0;
     float x[PER];
@@ -515,7 +543,10 @@ __global__ __launch_bounds__(SMP_WG) void k_smp_events(const float *logits, int6
 #pragma unroll
                 for (int q = 0; q + h < LB; q += 2 * h)
                     if (s0 + 16 * (q + h) < b) wave_merge_top(l[q], l[q + h]);
-            wave_merge_top(acc, l[0]);
+            if (s0 == wave)                            // the first batch
+#pragma unroll
+                for (int r = 0; r < R; r++) acc[r] = l[0][r];
+            else wave_merge_top(acc, l[0]);
         }
         wg_merge_top(acc, lds);
         if (wave == 0) wave_put(pb, acc);
@@ -529,8 +560,6 @@ __global__ __launch_bounds__(SMP_WG) void k_smp_events(const float *logits, int6
         const uint32_t kx = fkey(x[j]);
         key[j] = (b > 0 ? kx > tkey : x[j] > -__builtin_inff()) ? kx : 0u;
     }
-    // at most 64 candidates (every block but the first, for typical
-    // logits): one wave takes them in index order, one per lane
     int32_t *cc = ecnt;
 #pragma unroll
     for (int j = 0; j < PER; j++) {
@@ -546,25 +575,67 @@ __global__ __launch_bounds__(SMP_WG) void k_smp_events(const float *logits, int6
             if (lane >= o) inc += y;
         }
         if (lane < 16 * PER) cc[lane] = inc - c;
-        if (lane == 63) ncand_sh = inc;
+        if (lane == 63) sh.ncand = inc;
     }
     __syncthreads();
-    const int32_t ncand = ncand_sh;
-    if (ncand <= 64) {                                 // uniform
+    const int32_t ncand = sh.ncand;
+    if (ncand <= SMP_CAND) {                           // uniform; the candidates side by side, in index order
 #pragma unroll
         for (int j = 0; j < PER; j++) {
             const uint64_t m = __ballot(key[j] != 0u);
             if (key[j] != 0u) {
                 const int32_t pos = cc[wave * PER + j] + __builtin_popcountll(m & ((1ull << lane) - 1));
-                c1k[pos] = key[j];
-                c1i[pos] = (int32_t)(base + 64 * (wave * PER + j) + lane);
-                c1v[pos] = x[j];
+                sh.ck[pos] = key[j];
+                sh.ci[pos] = (int32_t)(base + 64 * (wave * PER + j) + lane);
+                sh.cv[pos] = x[j];
             }
         }
         __syncthreads();
+    }
+    if (ncand > 64 && ncand <= SMP_CAND) {             // uniform: P threads a candidate
+        const int P = ncand <= 256 ? 4 : 2, c = tid / P, part = P == 4 ? 64 : 256;
+        const uint32_t kv = c < ncand ? sh.ck[c] : 0u;
+        int32_t cnt = 0;
+        const int32_t c0 = (tid & (P - 1)) * part, c1 = min(c, c0 + part);
+        for (int32_t o = c0; o < c1; o += 4) {         // earlier candidates >= the candidate
+            const uint4 w = *reinterpret_cast<const uint4 *>(&sh.ck[o]);
+            cnt += w.x >= kv;
+            cnt += (o + 1 < c1) & (w.y >= kv);
+            cnt += (o + 2 < c1) & (w.z >= kv);
+            cnt += (o + 3 < c1) & (w.w >= kv);
+        }
+        cnt += dpp_xor1(cnt);
+        if (P == 4) cnt += dpp_xor2(cnt);
+        bool ev = false;
+        if (c < ncand && (tid & (P - 1)) == 0 && sh.ci[c] >= k) {   // the initial fill never enters
+            int32_t before = 0;                        // of the top of P
+            if (b > 0)
+#pragma unroll
+                for (int step = 64 * R; step > 0; step >>= 1)
+                    if (before + step <= k && pb[before + step - 1] >= kv) before += step;
+            ev = before + cnt < k;
+        }
+        const uint64_t m = __ballot(ev);
+        if (lane == 0) ecnt[wave] = __builtin_popcountll(m);
+        __syncthreads();
+        int32_t pos = __builtin_popcountll(m & ((1ull << lane) - 1)), all = 0;
+#pragma unroll
+        for (int w = 0; w < 16; w++) {
+            const int32_t e = ecnt[w];
+            pos += w < wave ? e : 0;
+            all += e;
+        }
+        if (ev) {
+            ev_idx[base + pos] = sh.ci[c];
+            ev_val[base + pos] = sh.cv[c];
+        }
+        if (tid == 0) ev_n[b] = all;
+        return;
+    }
+    if (ncand <= 64) {                                 // one wave takes them, one per lane
         if (wave != 0) return;
-        const uint32_t kv = lane < ncand ? c1k[lane] : 0u;
-        const int32_t idx = lane < ncand ? c1i[lane] : 0;
+        const uint32_t kv = lane < ncand ? sh.ck[lane] : 0u;
+        const int32_t idx = lane < ncand ? sh.ci[lane] : 0;
         bool ev = false;
         int32_t cnt = 0;
         if (kv != 0u && idx >= k) {                    // the initial fill never enters
@@ -585,7 +656,7 @@ __global__ __launch_bounds__(SMP_WG) void k_smp_events(const float *logits, int6
         if (ev) {
             const int32_t pos = __builtin_popcountll(m & ((1ull << lane) - 1));
             ev_idx[base + pos] = idx;
-            ev_val[base + pos] = c1v[lane];
+            ev_val[base + pos] = sh.cv[lane];
         }
         if (lane == 0) ev_n[b] = __builtin_popcountll(m);
         return;
@@ -640,21 +711,22 @@ __global__ __launch_bounds__(SMP_WG) void k_smp_events(const float *logits, int6
         wave_lds_sync();
         const uint32_t kv = key[j];
         const int64_t idx = base + 64 * (wave * PER + j) + lane;
-        bool ev = false;
         int32_t cnt = 0;                               // leading entries of the top >= v
-        if (kv != 0u && idx >= k) {                    // the initial fill never enters
+        if (kv != 0u) {
 #pragma unroll
             for (int step = 64 * R; step > 0; step >>= 1)
                 if (cnt + step <= k && my[cnt + step - 1] >= kv) cnt += step;
-            ev = cnt < k;
         }
-        if (__ballot(ev)) {                            // plus the earlier lanes of the sub-chunk
-            for (int l2 = 0; l2 < 63; l2++) {
-                const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int32_t)kv, l2);
-                cnt += (l2 < lane) & (o >= kv);
-            }
-            ev = ev && cnt < k;
+        // plus the earlier lanes of the sub-chunk. Only those whose count so
+        // far is below k matter: a larger one would have k before v as well.
+        uint64_t pass = __ballot(kv != 0u && cnt < k);
+        while (pass) {
+            const int l2 = __builtin_ctzll(pass);
+            pass &= pass - 1;
+            const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int32_t)kv, l2);
+            cnt += (l2 < lane) & (o >= kv);
         }
+        const bool ev = kv != 0u && idx >= k && cnt < k;   // the initial fill never enters
         wave_lds_sync();                               // the slot is rewritten for the next sub-chunk
         const uint64_t m = __ballot(ev);
         evf |= (int32_t)ev << j;
@@ -684,9 +756,19 @@ __global__ __launch_bounds__(SMP_WG) void k_smp_events(const float *logits, int6
     }
 }
 
+template <int PER, int R>
+__global__ __launch_bounds__(SMP_WG) void k_smp_events(const float *logits, int64_t n, int32_t k,
+                                                       const float *tops, int32_t *ev_idx, float *ev_val,
+                                                       int32_t *ev_n) {
+    __shared__ EvLds<R> sh;
+    const int64_t base = smp_base(blockIdx.x, PER);
+    if (PER > 1 && blockIdx.x < PER) events_body<1, R>(logits, n, k, tops, ev_idx, ev_val, ev_n, base, sh);
+    else events_body<PER, R>(logits, n, k, tops, ev_idx, ev_val, ev_n, base, sh);
+}
+
 struct SmpArgs {
     float temperature, top_p, min_p;
-    int32_t k, sb, nblk;
+    int32_t k, per, nblk;
 };
 
 __device__ __forceinline__ uint64_t rotl64(uint64_t x, int s) { return (x << s) | (x >> (64 - s)); }
@@ -727,7 +809,7 @@ __device__ __forceinline__ float readlane_f(float v, int32_t l) {
 }
 
 // The events of positions [e0, e0 + 64) as lane values (idx -1 past the end).
-__device__ __forceinline__ void gather_events(const int32_t *off, int32_t nblk, int32_t sb, int32_t e0,
+__device__ __forceinline__ void gather_events(const int32_t *off, int32_t nblk, int32_t per, int32_t e0,
                                               int32_t total, const int32_t *ev_idx, const float *ev_val,
                                               int32_t &gi, float &gv) {
     const int32_t e = e0 + (int32_t)threadIdx.x;
@@ -740,7 +822,7 @@ __device__ __forceinline__ void gather_events(const int32_t *off, int32_t nblk, 
             if (off[mid] <= e) lo = mid;
             else hi = mid;
         }
-        const int64_t a = (int64_t)lo * sb + (e - off[lo]);
+        const int64_t a = smp_base(lo, per) + (e - off[lo]);
         gi = ev_idx[a];
         gv = ev_val[a];
     }
@@ -808,25 +890,30 @@ __device__ void chain_literal(float *val, int32_t *idx, int32_t filled, const Sm
 }
 
 // ---- the slots and the pick ------------------------------------------------------
-// When the k fill values and the entering events are all distinct, the
-// replay has a closed form. Each event evicts the smallest slot value,
-// and what enters is larger than what leaves, so the evicted values come
-// out strictly increasing: the j-th event (in index order) evicts the
-// element of rank j among all N = k + events elements (the N - k
-// smallest are exactly the evicted ones, the k largest the survivors).
-// That element sits in its own fill slot, or in the slot of the earlier
-// event that brought it in, so every event's slot follows from the slots
-// of earlier events. One workgroup ranks the elements (by counting for
-// N <= 1024, else a bitonic sort in LDS), resolves the slots in event
-// order (one wave, 64 at a time, pointer jumping inside each group) and
-// places the survivors. Ties (equal keys, -0 and +0 included), a NaN in
-// the fill or more than SMP_NMAX elements send it to the replay instead:
-// one wave replays the events in order on the k slots. Then the rest of
-// the chain: the softmax numerators, their sum in slot order and the
-// quotients (wave 0), the ranking of the probabilities (every thread),
+// The replay of the k fill values and the entering events has a closed form.
+// Each event evicts the smallest slot value (of equal ones, the first slot's)
+// and what enters is larger than what leaves, so the evicted values never
+// fall: the j-th event (in index order) evicts the element of rank j among
+// all N = k + events elements (the N - k smallest are exactly the evicted
+// ones, the k largest the survivors). That element sits in its own fill
+// slot, or in the slot of the earlier event that brought it in, so every
+// event's slot follows from the slots of earlier events. Equal values (-0
+// and +0 included) have a run of ranks. Once one of a run is evicted nothing
+// of its value enters any more, so the run's slots are known before its
+// first event, and its events take them from the lowest up. One workgroup
+// ranks the elements (by buckets; a sort in registers or LDS where the values
+// crowd), resolves the slots (pointer jumping over the events between two runs,
+// then a run) and places the survivors. A NaN in the fill or more than SMP_NMAX elements send it to the
+// replay instead: one wave replays the events in order on the k slots. Then
+// the rest of the chain: the softmax numerators, their sum in slot order and
+// the quotients (wave 0), the ranking of the probabilities (every thread),
 // the cut and the pick (wave 0), and the masked ids get their saved values
-// back.
+// back. A tie among 2000 elements is common (two equal fp32 logits: one call
+// in three at vocabulary 248320, top-k 256); sent to the replay, such a call
+// took 825 us against 120.
 constexpr int SMP_NMAX = 4096;
+constexpr int SMP_BUCKETS = 2 * SMP_WG;                // of the elements' ranking
+constexpr int SMP_CROWD = 32;                          // elements in a bucket at most
 
 // One level of wg_sort_keys: waves w with w % 2l == 0 merge wave w + l's
 // list into theirs (exchanged through ex).
@@ -878,12 +965,16 @@ __global__ __launch_bounds__(SMP_WG) void k_smp_pick(float *logits, int64_t n, S
     __shared__ float sval[SMP_NMAX];
     __shared__ int32_t sid[SMP_NMAX];
     __shared__ int32_t byr[SMP_NMAX];                  // element of each rank; then the events' slots
+    int32_t *const lnk = reinterpret_cast<int32_t *>(skey);   // the events' links, once the ranks are known
+    __shared__ uint64_t eqb[SMP_NMAX / 64];            // bit r: ranks r and r + 1 have equal keys
     __shared__ uint64_t buf[SMP_NMAX];                 // (key << 32 | element), for the sort
     __shared__ __align__(16) float val[SMP_KMAX];      // the slots: values, then probabilities
     __shared__ int32_t idx[SMP_KMAX];
     __shared__ float sp[SMP_KMAX];                     // probabilities in sorted order
     __shared__ int32_t si[SMP_KMAX];
     __shared__ int32_t total_sh, nanf_sh, done_sh;
+    __shared__ uint32_t hist[SMP_BUCKETS], wtot[16];
+    __shared__ float red[32];
     const int tid = threadIdx.x, lane = tid & 63;
     const int32_t k = a.k, nblk = a.nblk;
     const int32_t filled = (int32_t)(n < k ? n : k);
@@ -927,29 +1018,118 @@ __global__ __launch_bounds__(SMP_WG) void k_smp_pick(float *logits, int64_t n, S
             if (off[mid] <= j) lo = mid;
             else hi = mid;
         }
-        return (int64_t)lo * a.sb + (j - off[lo]);
+        return smp_base(lo, a.per) + (j - off[lo]);
     };
     // the closed form applies: no NaN in the fill, events to place, room
-    bool closed = !nan_in_fill && total > 0 && N <= SMP_NMAX;
+    const bool closed = !nan_in_fill && total > 0 && N <= SMP_NMAX;
+    bool runs = false;                                 // equal keys among the elements
     if (closed) {                                      // uniform
-        for (int32_t e = tid; e < N; e += SMP_WG) {
-            float x;
-            int32_t id;
-            if (e < k) {
-                x = logits[e];
-                id = e;
-            } else {
-                const int64_t at = locate(e - k);
-                x = ev_val[at];
-                id = ev_idx[at];
+        constexpr int EU = SMP_NMAX / SMP_WG;          // elements per thread
+        int eq = 0;
+        float lo = __builtin_inff(), hi = -__builtin_inff();
+#pragma unroll
+        for (int u = 0; u < EU; u++) {
+            const int32_t e = tid + u * SMP_WG;
+            if (e < N) {
+                float x;
+                int32_t id;
+                if (e < k) {
+                    x = logits[e];
+                    id = e;
+                } else {
+                    const int64_t at = locate(e - k);
+                    x = ev_val[at];
+                    id = ev_idx[at];
+                }
+                skey[e] = fkey(x);
+                sval[e] = x;
+                sid[e] = id;
+                byr[e] = -1;
+                if (fabsf(x) < __builtin_inff()) {
+                    lo = fminf(lo, x);
+                    hi = fmaxf(hi, x);
+                }
             }
-            skey[e] = fkey(x);
-            sval[e] = x;
-            sid[e] = id;
+        }
+        lo = -wave_max(-lo);
+        hi = wave_max(hi);
+        if (lane == 0) {
+            red[tid >> 6] = lo;
+            red[16 + (tid >> 6)] = hi;
+        }
+        hist[tid] = hist[SMP_WG + tid] = 0;
+        __syncthreads();
+        // Ranks by buckets of equal width between the smallest and the
+        // largest value (about one element each: the entering values spread
+        // over the range), the order inside a bucket by comparing. A sort of
+        // 2000 elements and the binary searches in it took 11.6 us, this
+        // 3 us. Values that crowd into few buckets take the sorts below.
+        lo = red[lane & 15];
+        hi = red[16 + (lane & 15)];
+        lo = -wave_max(-lo);
+        hi = wave_max(hi);
+        const float scale = (float)(SMP_BUCKETS - 1) / __fsub_rn(hi, lo);
+        int32_t eb[EU], eo[EU];                        // an element's bucket; its place there
+#pragma unroll
+        for (int u = 0; u < EU; u++) {
+            const int32_t e = tid + u * SMP_WG;
+            eb[u] = eo[u] = 0;
+            if (e < N) {
+                const float f = __fmul_rn(__fsub_rn(sval[e], lo), scale);   // never falls as the value grows
+                eb[u] = !(f > 0.0f) ? 0 : f < (float)(SMP_BUCKETS - 1) ? (int32_t)f : SMP_BUCKETS - 1;
+                eo[u] = (int32_t)atomicAdd(&hist[eb[u]], 1u);
+            }
         }
         __syncthreads();
-        int tie = 0;
-        if (N <= 2 * SMP_WG) {                         // sorted in registers; ranks by binary search
+        const uint32_t h0 = hist[2 * tid], h1 = hist[2 * tid + 1];
+        uint32_t incl = h0 + h1;                       // inclusive scan: the wave, then the waves
+        incl += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)incl, 0x111, 0xF, 0xF, true);   // row_shr
+        incl += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)incl, 0x112, 0xF, 0xF, true);
+        incl += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)incl, 0x114, 0xF, 0xF, true);
+        incl += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)incl, 0x118, 0xF, 0xF, true);
+        incl += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)incl, 0x142, 0xA, 0xF, true);   // row_bcast
+        incl += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)incl, 0x143, 0xC, 0xF, true);
+        if (lane == 63) wtot[tid >> 6] = incl;
+        const bool crowded = __syncthreads_or(h0 > SMP_CROWD || h1 > SMP_CROWD);
+        if (!crowded) {
+            uint32_t before = incl - h0 - h1;
+#pragma unroll
+            for (int w = 0; w < 16; w++) before += w < (tid >> 6) ? wtot[w] : 0u;
+            hist[2 * tid] = before;                    // the buckets' starts
+            hist[2 * tid + 1] = before + h0;
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < EU; u++) {
+                const int32_t e = tid + u * SMP_WG;
+                if (e < N) buf[hist[eb[u]] + eo[u]] = ((uint64_t)skey[e] << 32) | (uint32_t)e;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < EU; u++) {
+                const int32_t e = tid + u * SMP_WG;
+                if (e < N) {
+                    const uint64_t mine = ((uint64_t)skey[e] << 32) | (uint32_t)e;
+                    const int32_t s0 = (int32_t)hist[eb[u]];
+                    const int32_t s1 = eb[u] + 1 < SMP_BUCKETS ? (int32_t)hist[eb[u] + 1] : N;
+                    int32_t r = s0;
+                    for (int32_t i = s0; i < s1; i++) {
+                        const uint64_t o = buf[i];
+                        r += o < mine;
+                        eq |= (o >> 32) == (mine >> 32) && o != mine;
+                    }
+                    byr[r] = e;
+                }
+            }
+            runs = __syncthreads_or(eq);
+            if (runs) {
+                for (int32_t r0 = tid & ~63; r0 < N; r0 += SMP_WG) {   // whole waves
+                    const int32_t r = min(r0 + lane, N - 1), r1 = min(r + 1, N - 1);
+                    const uint64_t m = __ballot(r0 + lane + 1 < N && skey[byr[r]] == skey[byr[r1]]);
+                    if (lane == 0) eqb[r0 >> 6] = m;
+                }
+                __syncthreads();
+            }
+        } else if (N <= 2 * SMP_WG) {                  // sorted in registers; ranks by binary search
             uint32_t *sorted = reinterpret_cast<uint32_t *>(buf);   // 2048 keys, then the exchange area
             uint32_t *ex = sorted + 2 * SMP_WG;
             if (N <= SMP_WG) wg_sort_keys<1>(skey, N, ex, sorted);
@@ -960,8 +1140,18 @@ __global__ __launch_bounds__(SMP_WG) void k_smp_pick(float *logits, int64_t n, S
                 int32_t pos = 0;                       // keys above kv
                 for (int32_t step = 2 * SMP_WG; step > 0; step >>= 1)
                     if (pos + step <= N && sorted[pos + step - 1] > kv) pos += step;
-                tie |= pos + 1 < N && sorted[pos + 1] == kv;   // another key equal to kv
-                byr[N - 1 - pos] = e;
+                if (pos + 1 < N && sorted[pos + 1] == kv) {   // a run: its ranks one element each, in any order
+                    int32_t r = N - 1 - pos;
+                    while (atomicCAS(&byr[r], -1, e) != -1) r--;
+                } else {
+                    byr[N - 1 - pos] = e;
+                }
+            }
+            for (int32_t r0 = tid & ~63; r0 < N; r0 += SMP_WG) {   // whole waves
+                const int32_t r = r0 + lane;
+                const uint64_t m = __ballot(r + 1 < N && sorted[N - 1 - min(r, N - 1)] == sorted[max(N - 2 - r, 0)]);
+                if (lane == 0) eqb[r0 >> 6] = m;
+                eq |= m != 0;
             }
         } else {                                       // bitonic sort of (key, element), ascending
             int32_t P = 2;
@@ -983,41 +1173,75 @@ __global__ __launch_bounds__(SMP_WG) void k_smp_pick(float *logits, int64_t n, S
                     __syncthreads();
                 }
             }
-            for (int32_t r = tid; r < N; r += SMP_WG) {
-                byr[r] = (int32_t)(uint32_t)buf[r];
-                tie |= r > 0 && (buf[r] >> 32) == (buf[r - 1] >> 32);
+            for (int32_t r0 = tid & ~63; r0 < N; r0 += SMP_WG) {   // whole waves
+                const int32_t r = r0 + lane;
+                if (r < N) byr[r] = (int32_t)(uint32_t)buf[r];
+                const uint64_t m = __ballot(r + 1 < N && buf[min(r, N - 1)] >> 32 == buf[min(r + 1, N - 1)] >> 32);
+                if (lane == 0) eqb[r0 >> 6] = m;
+                eq |= m != 0;
             }
         }
-        closed = !__syncthreads_or(tie);               // ties leave the order to the replay
+        if (crowded) runs = __syncthreads_or(eq);
     }
     if (closed) {
-        if (tid < 64) {                                // event j's slot, in event order
-            for (int32_t c0 = 0; c0 < total; c0 += 64) {
-                const int32_t j = c0 + lane;
-                int32_t p = j < total ? byr[j] : 0;    // the element event j evicts
-                int32_t slot = p, d = -1;              // resolved slot, or the in-group event it waits on
-                if (j < total && p >= k) {
-                    if (p - k < c0) slot = byr[p - k];   // an earlier group: resolved already
-                    else d = p - k - c0;               // an earlier lane of this group
+        // Event j's slot. Between two runs the events' links (to the event
+        // that brought in the element they evict) are followed by pointer
+        // jumping over all of them at once: a link holds ~slot once known,
+        // and whatever a thread reads is a valid link of that event, older
+        // or newer, so the rounds need no copy. The runs in event order.
+        for (int32_t c0 = 0; c0 < total;) {            // uniform
+            int32_t c1 = total;
+            if (runs) {                                // the next run's start, from c0 on (no run spans c0)
+                const int32_t w = (c0 >> 6) + lane;
+                uint64_t m = w < (N + 63) >> 6 ? eqb[w] : 0;
+                if (lane == 0) m &= ~0ull << (c0 & 63);
+                const uint64_t some = __ballot(m != 0);   // 64 words: every rank
+                if (some) {
+                    const int32_t f = __builtin_ctzll(some);
+                    const int32_t bit = m ? (int32_t)__builtin_ctzll(m) : 0;
+                    c1 = min(total, (((c0 >> 6) + f) << 6) + __builtin_amdgcn_readlane(bit, f));
                 }
-                for (int it = 0; it < 6 && __ballot(d >= 0); it++) {   // pointer jumping inside the group
-                    const int32_t ts = __shfl(slot, d < 0 ? lane : d);
-                    const int32_t td = __shfl(d, d < 0 ? lane : d);
-                    if (d >= 0) {
-                        if (td < 0) {
-                            slot = ts;
-                            d = -1;
-                        } else {
-                            d = td;
+            }
+            if (c1 > c0) {
+                for (int32_t j = c0 + tid; j < c1; j += SMP_WG) {
+                    const int32_t p = byr[j];          // the element event j evicts
+                    lnk[j] = p < k ? ~p : p - k < c0 ? ~byr[p - k] : p - k;
+                }
+                __syncthreads();
+                for (;;) {
+                    int open = 0;
+                    for (int32_t j = c0 + tid; j < c1; j += SMP_WG) {
+                        const int32_t d = lnk[j];
+                        if (d >= 0) {
+                            int32_t t = lnk[d];
+                            if (t >= 0) t = lnk[t];
+                            lnk[j] = t;
+                            open |= t >= 0;
                         }
                     }
+                    if (!__syncthreads_or(open)) break;
                 }
-                wave_lds_sync();                       // every lane has read byr for this group
-                if (j < total) byr[j] = slot;
-                wave_lds_sync();
+                for (int32_t j = c0 + tid; j < c1; j += SMP_WG) byr[j] = ~lnk[j];
+                c0 = c1;
+            } else {                                   // a run of at most k elements, all in slots by now
+                int32_t g = 2;
+                while (eqb[(c0 + g - 1) >> 6] >> ((c0 + g - 1) & 63) & 1) g++;
+                for (int32_t i = tid; i < g; i += SMP_WG) {
+                    const int32_t p = byr[c0 + i];
+                    idx[i] = p;
+                    si[i] = p < k ? p : byr[p - k];
+                }
+                __syncthreads();
+                for (int32_t i = tid; i < g; i += SMP_WG) {
+                    const int32_t slot = si[i];
+                    int32_t r = c0;                    // by slot; past the evictions the survivors stay elements
+                    for (int32_t o = 0; o < g; o++) r += si[o] < slot;
+                    byr[r] = r < total ? slot : idx[i];
+                }
+                c0 += g;
             }
+            __syncthreads();
         }
-        __syncthreads();
         for (int32_t r = total + tid; r < N; r += SMP_WG) {   // the survivors into their slots
             const int32_t e = byr[r];
             const int32_t slot = e < k ? e : byr[e - k];
@@ -1048,9 +1272,9 @@ __global__ __launch_bounds__(SMP_WG) void k_smp_pick(float *logits, int64_t n, S
             slot_min(sv, k, mv, ms);
             int32_t gi, ni;
             float gv, nv;
-            gather_events(off, nblk, a.sb, 0, total, ev_idx, ev_val, gi, gv);
+            gather_events(off, nblk, a.per, 0, total, ev_idx, ev_val, gi, gv);
             for (int32_t e0 = 0; e0 < total; e0 += 64) {
-                gather_events(off, nblk, a.sb, e0 + 64, total, ev_idx, ev_val, ni, nv);   // next batch in flight
+                gather_events(off, nblk, a.per, e0 + 64, total, ev_idx, ev_val, ni, nv);   // next batch in flight
                 const int32_t cnt = total - e0 < 64 ? total - e0 : 64;
                 for (int32_t j = 0; j < cnt; j++) {
                     const float v = readlane_f(gv, j);
@@ -1241,8 +1465,8 @@ static int32_t sample_block(int64_t n, int32_t k) {
 
 size_t sample_scratch_bytes(int64_t n, int32_t k) {
     const int32_t sb = sample_block(n, k);
-    const int64_t nblk = (n + sb - 1) / sb;
-    return (size_t)nblk * sb * 8                       // event indices and values
+    const int64_t nblk = smp_blocks_of(n, sb / SMP_BLOCK);
+    return (size_t)((n + sb - 1) / sb) * sb * 8        // event indices and values
            + (size_t)nblk * (size_t)k * 4              // per-block top-k lists
            + (size_t)nblk * 4 * 2                      // event counts, NaN flags
            + (size_t)((n + SMP_BLOCK - 1) / SMP_BLOCK) * sizeof(ArgPart) + 256    // greedy partials
@@ -1253,15 +1477,16 @@ hipError_t launch_sample(float *logits, int64_t n, float temperature, int32_t k,
                          float penalty, int32_t window, uint64_t *rng, const int32_t *history, int32_t hist_n,
                          const int32_t *mask, int32_t n_mask, int32_t *token, void *scratch, hipStream_t s) {
     const int32_t sb = sample_block(n, k);
-    const int32_t nblk = (int32_t)((n + sb - 1) / sb);
+    const int32_t per = sb / SMP_BLOCK, nblk = smp_blocks_of(n, per);
+    const size_t cap = (size_t)((n + sb - 1) / sb) * sb;   // event slots: one per logit
     // checked before the first launch, so a refused call leaves the logits
     // untouched (the caller's n limit keeps both)
     if (nblk > SMP_KMAX || sb > SMP_SBMAX || n_mask < 0 || n_mask > 2) return hipErrorInvalidValue;
     uint8_t *p = static_cast<uint8_t *>(scratch);
     int32_t *ev_idx = reinterpret_cast<int32_t *>(p);
-    p += (size_t)nblk * sb * 4;
+    p += cap * 4;
     float *ev_val = reinterpret_cast<float *>(p);
-    p += (size_t)nblk * sb * 4;
+    p += cap * 4;
     float *tops = reinterpret_cast<float *>(p);
     p += (size_t)nblk * (size_t)k * 4;
     int32_t *ev_n = reinterpret_cast<int32_t *>(p);
@@ -1299,7 +1524,7 @@ hipError_t launch_sample(float *logits, int64_t n, float temperature, int32_t k,
                          : (sb == 1024 ? k_smp_events<1, 4> : sb == 2048 ? k_smp_events<2, 4> : k_smp_events<4, 4>);
     hipLaunchKernelGGL(blocks, dim3(nblk), dim3(SMP_WG), 0, s, logits, n, k, tops, nan_flag, pp);
     hipLaunchKernelGGL(events, dim3(nblk), dim3(SMP_WG), 0, s, logits, n, k, tops, ev_idx, ev_val, ev_n);
-    SmpArgs sa{temperature, top_p, min_p, k, sb, nblk};
+    SmpArgs sa{temperature, top_p, min_p, k, per, nblk};
     hipLaunchKernelGGL(k_smp_pick, dim3(1), dim3(SMP_WG), 0, s, logits, n, sa, ev_idx, ev_val, ev_n, nan_flag, rng,
                        token, mk, saved);
     return hipGetLastError();

@@ -112,6 +112,41 @@ def test_sample_every_logit_enters(lib, orc):
             check(lib, orc, logits, sp, orc.rng_seed(n), [], [], f"n={n}")
 
 
+@pytest.mark.parametrize("n", [300, 1500, 6000, 40000, 248320])
+@pytest.mark.parametrize("top_k", [1, 40, 256])
+def test_sample_tied_values(lib, orc, n, top_k):
+    """Equal logits among the entering elements: one pair, pairs placed
+    late, runs of many (rounded logits), runs at the k-th value, -inf fills,
+    and +0 beside -0; from a few elements to more than the register sort
+    holds."""
+    step(f"sample ties n={n} k={top_k}")
+    rng = np.random.default_rng(n + top_k)
+    sp = dict(temperature=0.9, top_k=top_k, top_p=1.0, min_p=0.0, repetition_penalty=1.0, repetition_window=0)
+    base = (rng.standard_normal(n) * 3).astype(np.float32)
+    rows = []
+    for s in (4, 64, 4096):
+        rows.append((np.round(base * s) / s).astype(np.float32))
+    pair = base.copy()
+    order = np.argsort(base)
+    pair[order[-1 - top_k // 2]] = pair[order[-2 - top_k // 2]]
+    rows.append(pair)
+    late = base.copy()
+    late[-(n // 8):] = late[: n // 8]                    # copies of early values, at the end
+    rows.append(late)
+    kth = base.copy()
+    kth[rng.integers(0, n, 9)] = np.sort(base)[-min(n, top_k)]
+    rows.append(kth)
+    fill = base.copy()
+    fill[: min(n, 2 * top_k)] = -np.inf                # a run of -inf in the fill
+    rows.append(fill)
+    zeros = np.where(base > 5, base, np.where(rng.integers(0, 2, n) > 0, np.float32(0.0), np.float32(-0.0)))
+    rows.append(zeros.astype(np.float32))
+    steps = np.repeat(np.linspace(-4, 4, max(1, n // 3)), 3)[:n].astype(np.float32)   # rising, three equal at a time
+    rows.append(np.concatenate([steps, base[: n - steps.size]]))
+    for i, logits in enumerate(rows):
+        check(lib, orc, logits, sp, orc.rng_seed(31 * n + i), [], [], f"ties n={n} k={top_k} row={i}")
+
+
 def test_sample_rejects_bad_arguments(lib):
     import torch
     from conftest import qk
