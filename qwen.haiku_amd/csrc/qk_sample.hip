@@ -972,6 +972,7 @@ __global__ __launch_bounds__(SMP_WG) void k_smp_pick(float *logits, int64_t n, S
     __shared__ int32_t idx[SMP_KMAX];
     __shared__ float sp[SMP_KMAX];                     // probabilities in sorted order
     __shared__ int32_t si[SMP_KMAX];
+    __shared__ int32_t ord[SMP_KMAX];                  // the slots by falling logit (closed form)
     __shared__ int32_t total_sh, nanf_sh, done_sh;
     __shared__ uint32_t hist[SMP_BUCKETS], wtot[16];
     __shared__ float red[32];
@@ -1247,6 +1248,7 @@ __global__ __launch_bounds__(SMP_WG) void k_smp_pick(float *logits, int64_t n, S
             const int32_t slot = e < k ? e : byr[e - k];
             val[slot] = sval[e];
             idx[slot] = sid[e];
+            ord[N - 1 - r] = slot;
         }
     } else {
         for (int32_t s_ = tid; s_ < filled; s_ += SMP_WG) {   // the fill
@@ -1366,9 +1368,20 @@ __global__ __launch_bounds__(SMP_WG) void k_smp_pick(float *logits, int64_t n, S
     __syncthreads();
     const bool done = done_sh != 0;
     // topk_sort_desc (slm/sampler.c:116-129) is a stable sort by
-    // descending value: rank = #greater + #equal in earlier slots; one
-    // slot per thread, the probabilities read four at a time
-    if (!done) {                                       // uniform; four threads per slot
+    // descending value. The closed form knows the slots by falling logit:
+    // probabilities that fall strictly along them are in that order (the
+    // usual case). Else rank = #greater + #equal in earlier slots.
+    bool ranked = false;
+    if (!done && closed) {                             // uniform
+        const float p = tid < filled ? val[ord[tid]] : 0.0f;
+        const float q = tid + 1 < filled ? val[ord[tid + 1]] : -1.0f;
+        ranked = !__syncthreads_or(tid < filled && !(p > q));
+        if (ranked && tid < filled) {
+            sp[tid] = p;
+            si[tid] = idx[ord[tid]];
+        }
+    }
+    if (!done && !ranked) {                            // uniform; four threads per slot, four values a read
         const int32_t sl = tid >> 2, t0 = (tid & 3) * 64;
         const int32_t nf4 = (filled + 3) & ~3, t1 = t0 + 64 < nf4 ? t0 + 64 : nf4;
         float v = 0.0f;
@@ -1403,17 +1416,24 @@ __global__ __launch_bounds__(SMP_WG) void k_smp_pick(float *logits, int64_t n, S
         // the pick's c) are one sequence of adds from 0 in sorted order, so
         // one pass keeps every partial sum (lane j % 64 of pre[j / 64]);
         // entries past filled add +0.
+        // Lane l's sum is lane l - 1's plus its own value: 63 rounds of a
+        // wave shift and an add settle them in order.
         float pre[SMP_Q];
-        float acc = 0.0f;
+        float acc = 0.0f;                              // the sum before the register, in every lane
 #pragma unroll
         for (int q = 0; q < SMP_Q; q++) {
             pre[q] = 0.0f;
-            if (q * 64 < filled)
+            if (q * 64 < filled) {
+                float c = __fadd_rn(acc, sq[q]);       // right in lane 0
 #pragma unroll
-                for (int l = 0; l < 64; l++) {
-                    acc = __fadd_rn(acc, readlane_f(sq[q], l));
-                    pre[q] = lane == l ? acc : pre[q];
+                for (int l = 1; l < 64; l++) {
+                    const float b = __int_as_float(__builtin_amdgcn_update_dpp(
+                        __float_as_int(acc), __float_as_int(c), 0x138, 0xF, 0xF, false));   // wave_shr:1
+                    c = __fadd_rn(b, sq[q]);
                 }
+                pre[q] = c;
+                acc = readlane_f(c, 63);
+            }
         }
         // the first j meeting a per-lane predicate, or -1
         auto first = [&](auto pred) -> int32_t {
