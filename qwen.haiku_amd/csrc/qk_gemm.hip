@@ -1442,6 +1442,101 @@ __global__ __launch_bounds__(512) void k_gemm_q80(const uint8_t *__restrict__ w,
     }
 }
 
+// The same product for few outputs (the model's 16-row ssm_alpha and
+// ssm_beta): a workgroup owns 16 weight rows x 8 tokens, so a short prompt
+// still has a workgroup for every 8 tokens. Lane (token, slot) holds the
+// slot's fp32 chain of two rows; a slot's four bytes of a block are one
+// v_dot4. 32 blocks (the whole of k = 1024) are staged at once, slot-major,
+// so a lane reads four blocks with one LDS read and the loads of a step are
+// one trip to memory instead of four. MFMA tiles would be half empty here
+// and their 32 x 32 outputs leave 11 workgroups at 333 tokens.
+#define G8S_R 16
+#define G8S_T 8
+#define G8S_KB 32
+#define G8S_LD (G8S_KB + 4)           // LDS row stride (dwords): rows on different banks
+
+template <bool FUSED>
+__global__ __launch_bounds__(512) void k_gemm_q80_few(const uint8_t *__restrict__ w, int64_t n, int nb,
+                                                      const uint8_t *__restrict__ xq, int64_t m,
+                                                      float *__restrict__ y) {
+    // rows 0-15: weights, 16-23: tokens
+    __shared__ __align__(16) uint32_t qs[G8S_R + G8S_T][8][G8S_LD];
+    __shared__ __align__(16) float ds[G8S_R + G8S_T][G8S_LD];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t r0 = (int64_t)blockIdx.x * G8S_R, t0 = (int64_t)blockIdx.y * G8S_T;
+    const int rowb = nb * Q80_BYTES;
+    const int nrows = (n - r0 < G8S_R) ? (int)(n - r0) : G8S_R;
+    const int mrows = (m - t0 < G8S_T) ? (int)(m - t0) : G8S_T;
+    const uint8_t *wt = w + r0 * rowb, *xt = xq + t0 * rowb;
+    // buffers as in k_gemm_q80: rows past n and tokens past m read zeros
+    const int wmis = (int)(reinterpret_cast<uintptr_t>(wt) & 3u), xmis = (int)(reinterpret_cast<uintptr_t>(xt) & 3u);
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t *>(wt - wmis), 0, (wmis + nrows * rowb + 3) & ~3, 0x00020000);
+    const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t *>(xt - xmis), 0, (xmis + mrows * rowb + 3) & ~3, 0x00020000);
+    // staging: block tid % 32 of weight row tid / 32, and (threads 0-255) of token tid / 32
+    const int sb = tid & (G8S_KB - 1), sr = tid / G8S_KB;
+    Q80Raw rw, rx;
+    auto load_step = [&](int b0) __attribute__((always_inline)) {
+        if (b0 + sb >= nb) return;
+        load_q80(rw, wr, wmis + sr * rowb + (b0 + sb) * Q80_BYTES);
+        if (sr < G8S_T) load_q80(rx, xr, xmis + sr * rowb + (b0 + sb) * Q80_BYTES);
+    };
+    auto put = [&](const Q80Raw &r, int row) __attribute__((always_inline)) {
+        const uint32_t v[9] = {r.a.x, r.a.y, r.a.z, r.a.w, r.b.x, r.b.y, r.b.z, r.b.w, r.c};
+#pragma unroll
+        for (int i = 0; i < 8; i++) qs[row][i][sb] = __builtin_amdgcn_alignbyte(v[i + 1], v[i], r.sh);
+        ds[row][sb] = h2f(r.d);
+    };
+    load_step(0);
+    const int sl = lane & 7, tt = lane >> 3;
+    float acc[2] = {0.0f, 0.0f};
+    for (int b0 = 0; b0 < nb; b0 += G8S_KB) {
+        const int kn = (nb - b0 < G8S_KB) ? nb - b0 : G8S_KB;
+        lds_barrier();                                   // previous step's reads done
+        if (sb < kn) {
+            put(rw, sr);
+            if (sr < G8S_T) put(rx, G8S_R + sr);
+        }
+        if (b0 + G8S_KB < nb) load_step(b0 + G8S_KB);    // next step in flight during compute
+        lds_barrier();
+#pragma unroll
+        for (int g = 0; g < G8S_KB; g += 4) {
+            if (g >= kn) break;                          // uniform
+            const uint4 xv = *reinterpret_cast<const uint4 *>(&qs[G8S_R + tt][sl][g]);
+            const float4 dv = *reinterpret_cast<const float4 *>(&ds[G8S_R + tt][g]);
+            const uint32_t xb[4] = {xv.x, xv.y, xv.z, xv.w};
+            const float dx[4] = {dv.x, dv.y, dv.z, dv.w};
+#pragma unroll
+            for (int r = 0; r < 2; r++) {
+                const uint4 wv = *reinterpret_cast<const uint4 *>(&qs[2 * wave + r][sl][g]);
+                const float4 ev = *reinterpret_cast<const float4 *>(&ds[2 * wave + r][g]);
+                const uint32_t wb[4] = {wv.x, wv.y, wv.z, wv.w};
+                const float dw[4] = {ev.x, ev.y, ev.z, ev.w};
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    if (g + i >= kn) break;              // uniform
+                    const int32_t p = dot4(wb[i], xb[i], 0);
+                    const float sc = __fmul_rn(dw[i], dx[i]);
+                    if (FUSED) acc[r] = __builtin_fmaf((float)p, sc, acc[r]);
+                    else acc[r] = __fadd_rn(acc[r], __fmul_rn((float)sum8(p), sc));
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        float a = acc[r];
+        if (FUSED) {                                     // ((a0+a4)+(a1+a5)) + ((a2+a6)+(a3+a7)) in slot 0
+            a = __fadd_rn(a, swz_xor4(a));
+            a = __fadd_rn(a, swz_xor1(a));
+            a = __fadd_rn(a, swz_xor2(a));
+        }
+        const int64_t t = t0 + tt, row = r0 + 2 * wave + r;
+        if (sl == 0 && t < m && row < n) y[t * n + row] = a;
+    }
+}
+
 hipError_t launch_gemm(int type, const uint8_t *w, int64_t n, int64_t k, const uint8_t *xq, int64_t m,
                        float *y, int fused, hipStream_t s) {
     if (type == 8) {
@@ -1450,6 +1545,15 @@ hipError_t launch_gemm(int type, const uint8_t *w, int64_t n, int64_t k, const u
         // 32 x 64 and 16 x 64 at M = 64..2048: 14.7 / 18.2 / 15.5 us at
         // M = 512, N = K = 1024)
         const dim3 grid((unsigned)((n + 31) / 32), (unsigned)((m + 31) / 32));
+        // 16 x 8 outputs a workgroup while those are at most 1024 (k = 1024:
+        // n = 16, m = 333 4.5 against 8.6 us, 2048 4.8 / 8.7, 8192 8.6 / 9.5;
+        // 512 x 256 8.7 / 9.4; beyond, the MFMA tiles are full)
+        const dim3 few((unsigned)((n + G8S_R - 1) / G8S_R), (unsigned)((m + G8S_T - 1) / G8S_T));
+        if ((uint64_t)few.x * ((m + G8S_T - 1) / G8S_T) <= 1024) {
+            if (fused) hipLaunchKernelGGL((k_gemm_q80_few<true>), few, dim3(512), 0, s, w, n, nb, xq, m, y);
+            else hipLaunchKernelGGL((k_gemm_q80_few<false>), few, dim3(512), 0, s, w, n, nb, xq, m, y);
+            return hipGetLastError();
+        }
         if (fused) hipLaunchKernelGGL((k_gemm_q80<true, 32, 32>), grid, dim3(512), 0, s, w, n, nb, xq, m, y);
         else hipLaunchKernelGGL((k_gemm_q80<false, 32, 32>), grid, dim3(512), 0, s, w, n, nb, xq, m, y);
         return hipGetLastError();

@@ -220,6 +220,23 @@ def test_matmul_gemm(tier, orc, wtype, n, k, m, epi, t):
     assert_bits_equal(got, want, f"gemm {wtype} {m}x{n}x{k}")
 
 
+@pytest.mark.parametrize("n,k,m", [(15, 32, 7), (17, 1024, 9), (16, 1056, 8), (31, 1088, 23), (2, 4160, 1),
+                                   (512, 64, 256), (513, 64, 257), (513, 2080, 260), (1000, 96, 1001), (4100, 32, 130)])
+@pytest.mark.parametrize("epi,t", EPI_TIERS)
+def test_matmul_q80_splits(tier, orc, n, k, m, epi, t):
+    """Q8_0 on both sides of the line between 16 x 8 outputs a workgroup
+    (up to 1024 of them) and MFMA tiles: partial rows, tokens and steps."""
+    lib = tier
+    step(f"matmul Q8_0 splits n={n} k={k} m={m} tier={t}")
+    lib.set_tier(t)
+    w = synth.blocks(8, n, k, seed=m, tag=8)
+    w[-1, -32:] = 0x80                                 # quants of -128
+    x = synth.activations(m, k, seed=m + 1)
+    xq = orc.quantize_for(8, x)
+    got = host(lib.matmul(8, dev(w), n, k, dev(xq), m))
+    assert_bits_equal(got, orc.matmul_xq(8, w, n, k, xq, m, epi), f"gemm Q8_0 {m}x{n}x{k}")
+
+
 def test_matmul_gemm_m2048(lib, orc):
     step("matmul config 3 M=2048")
     n, k, m = 3584, 1024, 2048
