@@ -338,10 +338,10 @@ void k_gemm_planes(const uint8_t *__restrict__ wp, int64_t n, int nb, const uint
 template <int TYPE, bool FUSED, int S, bool PF>
 __global__ __launch_bounds__(64 * S) void k_gemm_planes_ks(const uint8_t *__restrict__ wp, int64_t n, int nb,
                                                         const uint8_t *__restrict__ xq, int64_t m,
-                                                        float *__restrict__ y) {
+                                                        float *__restrict__ y, int lsplit) {
     constexpr bool KQ = TYPE != 14;
     constexpr int CH = pl_chunk(TYPE);
-    static_assert(S == 4, "one staging pass covers four super-blocks");
+    static_assert(S == 4 || (S == 8 && PF), "256 threads stage four super-blocks in one pass");
     constexpr int VW = 16 / S;                         // outputs per lane each wave adds up
     __shared__ __attribute__((aligned(16))) int8_t sa[S][32][PL_LD];
     __shared__ __attribute__((aligned(16))) float st[S][16][64];    // the waves' terms, [wave][v][lane]
@@ -349,15 +349,19 @@ __global__ __launch_bounds__(64 * S) void k_gemm_planes_ks(const uint8_t *__rest
     __shared__ __attribute__((aligned(16))) float syd[S][32];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 31, h = lane >> 5;
-    const int64_t g = blockIdx.x, t0 = (int64_t)blockIdx.y * 32;
+    // 2^lsplit workgroups share a tile, each 32 >> lsplit of its rows: the
+    // other rows' lanes read past the buffer (zeros, no memory access)
+    const int64_t g = blockIdx.x >> lsplit, t0 = (int64_t)blockIdx.y * 32;
+    const bool mine = (col >> (5 - lsplit)) == (int)(blockIdx.x & ((1u << lsplit) - 1));
+    const int wlane = mine ? 16 * lane : 0x40000000;
     const int mrows = (m - t0 < 32) ? (int)(m - t0) : 32;
     const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint8_t *>(xq + t0 * nb * Q8K_BYTES), 0, mrows * nb * Q8K_BYTES, 0x00020000);
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint8_t *>(wp + g * nb * (int64_t)CH), 0, nb * CH, 0x00020000);
-    // staging: thread t stages eighth e = t % 8 of token t / 8 for the
-    // round's four super-blocks
-    const int at = tid >> 3, ae = tid & 7;
+    // staging: thread t stages eighth e = t % 8 of token t / 8 (mod 32) for
+    // four of the round's super-blocks, qb ..
+    const int at = (tid >> 3) & 31, ae = tid & 7, qb = 4 * (tid >> 8);
     float sum[VW];
 #pragma unroll
     for (int b = 0; b < VW; b++) sum[b] = 0.0f;
@@ -375,17 +379,17 @@ __global__ __launch_bounds__(64 * S) void k_gemm_planes_ks(const uint8_t *__rest
         const int sb = r + wave;
 #pragma unroll
         for (int q = 0; q < 16; q++) {
-            const auto v = __builtin_amdgcn_raw_buffer_load_b128(wr, 16 * lane, sb * CH + 1024 * q, 0);
+            const auto v = __builtin_amdgcn_raw_buffer_load_b128(wr, wlane, sb * CH + 1024 * q, 0);
             o.bq[q] = p4i{(int)v[0], (int)v[1], (int)v[2], (int)v[3]};
         }
-        if (KQ) o.bmn = __builtin_bit_cast(p8h, __builtin_amdgcn_raw_buffer_load_b128(wr, 16 * lane, sb * CH + PL_PLANES, 0));
+        if (KQ) o.bmn = __builtin_bit_cast(p8h, __builtin_amdgcn_raw_buffer_load_b128(wr, wlane, sb * CH + PL_PLANES, 0));
         const auto sc = __builtin_amdgcn_raw_buffer_load_b64(wr, 8 * col, sb * CH + pl_scal_off(TYPE), 0);
         o.scw[0] = sc[0], o.scw[1] = sc[1];
     };
     auto load_a = [&](Ops &o, int r) {
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            const int sq = r + q;
+            const int sq = r + qb + q;
             const int of = at * nb * Q8K_BYTES + (sq < nb ? sq : nb - 1) * Q8K_BYTES;
             o.ar[q].q0 = bl128(xr, of + 4 + 32 * ae);
             o.ar[q].q1 = bl128(xr, of + 20 + 32 * ae);
@@ -401,7 +405,7 @@ __global__ __launch_bounds__(64 * S) void k_gemm_planes_ks(const uint8_t *__rest
         if (r > 0) pl_barrier();                       // the previous round's reads of st done
 #pragma unroll
         for (int q = 0; q < 4; q++) {
-            const int qq = q;
+            const int qq = qb + q;
             *(QK_LDS uint4 *)&sa[qq][at][32 * ae] = o.ar[q].q0;
             *(QK_LDS uint4 *)&sa[qq][at][32 * ae + 16] = o.ar[q].q1;
             if (KQ) {
@@ -474,10 +478,10 @@ __global__ __launch_bounds__(64 * S) void k_gemm_planes_ks(const uint8_t *__rest
             p8h bmn;
     #pragma unroll
             for (int q = 0; q < 16; q++) {
-                const auto v = __builtin_amdgcn_raw_buffer_load_b128(wr, 16 * lane, sb * CH + 1024 * q, 0);
+                const auto v = __builtin_amdgcn_raw_buffer_load_b128(wr, wlane, sb * CH + 1024 * q, 0);
                 bq[q] = p4i{(int)v[0], (int)v[1], (int)v[2], (int)v[3]};
             }
-            if (KQ) bmn = __builtin_bit_cast(p8h, __builtin_amdgcn_raw_buffer_load_b128(wr, 16 * lane, sb * CH + PL_PLANES, 0));
+            if (KQ) bmn = __builtin_bit_cast(p8h, __builtin_amdgcn_raw_buffer_load_b128(wr, wlane, sb * CH + PL_PLANES, 0));
             const auto sc = __builtin_amdgcn_raw_buffer_load_b64(wr, 8 * col, sb * CH + pl_scal_off(TYPE), 0);
             const float wd = __uint_as_float(sc[0]), wdm = __uint_as_float(sc[1]);
             // the round's activations
@@ -552,7 +556,7 @@ __global__ __launch_bounds__(64 * S) void k_gemm_planes_ks(const uint8_t *__rest
         }
     }
     const int64_t row = g * 32 + col;
-    if (row < n) {
+    if (mine && row < n) {
 #pragma unroll
         for (int b = 0; b < VW; b++) {
             const int64_t t = t0 + pl_tok(VW * wave + b, h);
@@ -568,18 +572,37 @@ static void launch_planes(const uint8_t *wp, int64_t n, int nb, const uint8_t *x
         // Q6_K: operands a round ahead when the tiles fit one workgroup per
         // CU (1024 x 3584: M = 128 11.3 -> 10.4 us; Q5_K and more tiles
         // were slower with it)
-        const dim3 grid((unsigned)((n + 31) / 32), (unsigned)((m + 31) / 32));
-        const bool pf = (uint64_t)grid.x * grid.y <= 256;
-#define QK_PLKS(F, P) hipLaunchKernelGGL((k_gemm_planes_ks<TYPE, F, 4, P>), grid, dim3(256), 0, s, wp, n, nb, xq, m, y)
+        dim3 grid((unsigned)((n + 31) / 32), (unsigned)((m + 31) / 32));
+        const uint64_t tiles = (uint64_t)grid.x * grid.y;
+        const bool pf = tiles <= 256;
+        int lsplit = 0;
+#define QK_PLKS(F, S, P) \
+    hipLaunchKernelGGL((k_gemm_planes_ks<TYPE, F, S, P>), grid, dim3(64 * S), 0, s, wp, n, nb, xq, m, y, lsplit)
+        // There, eight super-blocks a round where that halves the rounds or
+        // nearly so (planes from HBM: Q5_K 1024 x 2048 at M = 23 5.8 -> 5.2
+        // us, 768 x 1536 at M = 300 5.8 -> 5.2, Q6_K 2560 x 7168 at M = 33
+        // 18.4 -> 17.0; nine or ten super-blocks 6.8 -> 7.1, so not those).
+        // Beyond twelve the planes of a tile are 230 KB and more, and up to
+        // four workgroups share them, 8 rows (128-byte pieces) each, while
+        // that leaves one workgroup per CU (Q6_K 1024 x 3584: M = 23 10.4 ->
+        // 8.8 us, 128 10.3 -> 9.0, 256 10.4 -> 9.8; with few super-blocks the
+        // shared activations cost as much: 1024 x 1024 3.8 -> 3.9).
+        if (pf && nb > 4 && (nb <= 8 || nb > 12)) {
+            if (nb > 12) lsplit = tiles <= 64 ? 2 : tiles <= 128 ? 1 : 0;
+            grid.x <<= lsplit;
+            if (fused) QK_PLKS(true, 8, true);
+            else QK_PLKS(false, 8, true);
+            return;
+        }
         if constexpr (TYPE == 14) {
             if (pf) {
-                if (fused) QK_PLKS(true, true);
-                else QK_PLKS(false, true);
+                if (fused) QK_PLKS(true, 4, true);
+                else QK_PLKS(false, 4, true);
                 return;
             }
         }
-        if (fused) QK_PLKS(true, false);
-        else QK_PLKS(false, false);
+        if (fused) QK_PLKS(true, 4, false);
+        else QK_PLKS(false, 4, false);
 #undef QK_PLKS
     } else {
         const dim3 grid((unsigned)(((n + 31) / 32 + 3) / 4), (unsigned)((m + 63) / 64));
@@ -594,8 +617,8 @@ static void launch_planes(const uint8_t *wp, int64_t n, int nb, const uint8_t *x
 // at M = 512 15.1 us against 22.4 for k_gemm_planes, Q5_K 2048 x 1024 at
 // M = 512 8.3 / 12.2); beyond, 64-token tiles walk the super-blocks
 // (Q6_K at M = 2048 28.0 / 37.6, Q5_K 2048 x 1024 at M = 1024 11.0 /
-// 12.6). One token tile or four per wave, and eight waves per tile, were
-// slower everywhere.
+// 12.6). One token tile or four per wave were slower everywhere, eight waves
+// per tile wherever the tiles outnumber the CUs.
 hipError_t launch_gemm_planes(int type, const uint8_t *wp, int64_t n, int64_t k, const uint8_t *xq, int64_t m,
                               float *y, int fused, hipStream_t s) {
     const int nb = (int)(k / QK_K);

@@ -64,6 +64,25 @@ def test_matmul_planes(tier, orc, wtype, n, k, m, epi, t):
     assert_bits_equal(got, want, f"planes {wtype} {m}x{n}x{k}")
 
 
+# Four or eight super-blocks a round (5 .. 8 and past 12 of them, up to 256
+# tiles), a tile's rows over one, two or four workgroups (past 12; at most
+# 64 and 128 tiles), on both sides of each line, with partial tiles.
+@pytest.mark.parametrize("n,nb,m", [(40, 4, 5), (40, 5, 33), (70, 8, 9), (33, 9, 40), (65, 12, 3), (1, 13, 1),
+                                    (35, 13, 31), (1000, 13, 50), (1000, 14, 100), (4000, 13, 64), (4128, 13, 64),
+                                    (60, 17, 34), (2100, 5, 97)])
+@pytest.mark.parametrize("wtype", [12, 13, 14])
+@pytest.mark.parametrize("epi,t", EPI_TIERS)
+def test_matmul_planes_few_tiles(tier, orc, wtype, n, nb, m, epi, t):
+    lib, k = tier, 256 * nb
+    step(f"planes few tiles type={wtype} n={n} k={k} m={m} tier={t}")
+    lib.set_tier(t)
+    w = synth.blocks(wtype, n, k, seed=n + m, tag=wtype)
+    xq = orc.quantize_for(wtype, synth.activations(m, k, seed=m + 1))
+    planes = lib.pack_planes(wtype, dev(w), n, k)
+    got = host(lib.matmul_planes(wtype, planes, n, k, dev(xq), m))
+    assert_bits_equal(got, orc.matmul_xq(wtype, w, n, k, xq, m, epi), f"planes {wtype} {m}x{n}x{k}")
+
+
 def _extreme_blocks(wtype, n, k, seed):
     """Blocks whose folded weights reach the ends of the planes' range."""
     w = synth.blocks(wtype, n, k, seed=seed, tag=wtype)
