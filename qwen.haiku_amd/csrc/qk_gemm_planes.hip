@@ -618,11 +618,19 @@ static void launch_planes(const uint8_t *wp, int64_t n, int nb, const uint8_t *x
 // M = 512 8.3 / 12.2); beyond, 64-token tiles walk the super-blocks
 // (Q6_K at M = 2048 28.0 / 37.6, Q5_K 2048 x 1024 at M = 1024 11.0 /
 // 12.6). One token tile or four per wave were slower everywhere, eight waves
-// per tile wherever the tiles outnumber the CUs.
+// per tile wherever the tiles outnumber the CUs. The line moves with what
+// the last round of the first kernel's four waves leaves idle: three of
+// them with one super-block, so 768 tiles (Q5_K 6144 x 256 at M = 160 7.2
+// against 5.8 us, Q6_K 6.3 / 5.6; at 768 tiles 6.1 / 5.7 and 5.3 / 5.5);
+// none with four, so 1280 (Q5_K 4096 x 1024 at M = 290 10.8 / 12.2, Q6_K
+// 10.1 / 11.4; from 1536 equal), and Q6_K with three as well (8.3 / 9.3;
+// Q5_K 9.6 / 10.1 there but 9.4 / 9.1 at 1024 x 768, M = 1280). With two,
+// and from five on, the two meet near 1024 or within 6 % of each other.
 hipError_t launch_gemm_planes(int type, const uint8_t *wp, int64_t n, int64_t k, const uint8_t *xq, int64_t m,
                               float *y, int fused, hipStream_t s) {
     const int nb = (int)(k / QK_K);
-    const bool ks = (uint64_t)((n + 31) / 32) * (uint64_t)((m + 31) / 32) <= 1024 && (m + 31) / 32 <= 65535;
+    const int most = nb == 1 ? 768 : nb == 4 || (nb == 3 && type == 14) ? 1280 : 1024;
+    const bool ks = (uint64_t)((n + 31) / 32) * (uint64_t)((m + 31) / 32) <= (uint64_t)most && (m + 31) / 32 <= 65535;
     switch (type) {
         case 12: launch_planes<12>(wp, n, nb, xq, m, y, fused, ks, s); break;
         case 13: launch_planes<13>(wp, n, nb, xq, m, y, fused, ks, s); break;

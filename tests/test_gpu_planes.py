@@ -83,6 +83,23 @@ def test_matmul_planes_few_tiles(tier, orc, wtype, n, nb, m, epi, t):
     assert_bits_equal(got, orc.matmul_xq(wtype, w, n, k, xq, m, epi), f"planes {wtype} {m}x{n}x{k}")
 
 
+# Both sides of the line between super-blocks across waves and 64-token
+# tiles, where few super-blocks move it: 768 tiles with one, 1280 with four
+# (Q6_K: with three too).
+@pytest.mark.parametrize("n,nb,m", [(6144, 1, 100), (6150, 1, 100), (5110, 3, 250), (5130, 3, 250), (8190, 4, 130),
+                                    (8200, 4, 130)])
+@pytest.mark.parametrize("wtype", [13, 14])
+def test_matmul_planes_few_super_blocks(tier, orc, wtype, n, nb, m):
+    lib, k = tier, 256 * nb
+    step(f"planes few super-blocks type={wtype} n={n} k={k} m={m}")
+    w = synth.blocks(wtype, n, k, seed=n + m, tag=wtype)
+    xq = orc.quantize_for(wtype, synth.activations(m, k, seed=m + 1))
+    planes = lib.pack_planes(wtype, dev(w), n, k)
+    got = host(lib.matmul_planes(wtype, planes, n, k, dev(xq), m))
+    assert_bits_equal(got, orc.matmul_xq(wtype, w, n, k, xq, m, oracle.TIER_EPI[lib.tier()]),
+                      f"planes {wtype} {m}x{n}x{k}")
+
+
 def _extreme_blocks(wtype, n, k, seed):
     """Blocks whose folded weights reach the ends of the planes' range."""
     w = synth.blocks(wtype, n, k, seed=seed, tag=wtype)
