@@ -270,7 +270,7 @@ __global__ __launch_bounds__(256) void k_smp_argmax_final(float *logits, int64_t
 
 // ---- sampling path ------------------------------------------------------------
 // Blocks of sb logits (a power of two >= 1024, chosen by the launcher so
-// that nblk * k <= SMP_LIST_MAX). A NaN logit at an index >= k never
+// that ceil(n / sb) * k <= SMP_LIST_MAX). A NaN logit at an index >= k never
 // enters the slots and never compares >= anything, so it is read as -inf
 // here; a NaN among the first k (the initial fill) is flagged instead and
 // k_smp_pick then runs topk_collect literally.
@@ -1475,7 +1475,7 @@ __global__ __launch_bounds__(SMP_WG) void k_smp_pick(float *logits, int64_t n, S
 }
 
 // ---- launcher -------------------------------------------------------------------
-// Block size: the smallest power of two >= 1024 with nblk * k within the
+// Block size: the smallest power of two >= 1024 with ceil(n / sb) * k within the
 // LDS list budget (n <= QK_SAMPLE_MAX_N keeps it <= 4096 and nblk <= 256).
 static int32_t sample_block(int64_t n, int32_t k) {
     int32_t sb = 1024;
@@ -1534,7 +1534,7 @@ hipError_t launch_sample(float *logits, int64_t n, float temperature, int32_t k,
         hipLaunchKernelGGL(k_smp_argmax_final, dim3(1), dim3(256), 0, s, logits, n, part, ablk, token, mk, saved);
         return hipGetLastError();
     }
-    // (sb, list registers): sb <= 1024 * R, since nblk * k <= SMP_LIST_MAX
+    // (sb, list registers): sb <= 1024 * R, since ceil(n / sb) * k <= SMP_LIST_MAX
     const int R = smp_regs(k);
     auto blocks = R == 1 ? k_smp_blocks<1, 1>
                 : R == 2 ? (sb == 1024 ? k_smp_blocks<1, 2> : k_smp_blocks<2, 2>)
