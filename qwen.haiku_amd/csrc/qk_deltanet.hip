@@ -87,6 +87,13 @@ __device__ __forceinline__ float4 scale4(float4 v, float s) {
     return make_float4(__fmul_rn(v.x, s), __fmul_rn(v.y, s), __fmul_rn(v.z, s), __fmul_rn(v.w, s));
 }
 
+// The same for columns 4c .. of which `left` lie within the head dim: the
+// padding stays 0 where s is infinite or NaN.
+__device__ __forceinline__ float4 scale4(float4 v, float s, int left) {
+    const float4 p = scale4(v, s);
+    return make_float4(left > 0 ? p.x : 0.0f, left > 1 ? p.y : 0.0f, left > 2 ? p.z : 0.0f, left > 3 ? p.w : 0.0f);
+}
+
 __device__ __forceinline__ bool finite(float x) { return fabsf(x) < __builtin_inff(); }
 __device__ __forceinline__ bool finite4(float4 v) { return finite(v.x) && finite(v.y) && finite(v.z) && finite(v.w); }
 
@@ -295,7 +302,7 @@ __global__ __launch_bounds__(DN_WG) void k_dn_chunk(DnArgs a, DnScratch s) {
         if (part == 2) {
             B[dn_swz(t, c)] = r2[u];
         } else {
-            kr[u] = scale4(kr[u], bt[u]);              // K * beta
+            kr[u] = scale4(kr[u], bt[u], kd - 4 * c);  // K * beta
             B[dn_swz(t, c)] = kr[u];
         }
     }
@@ -306,7 +313,7 @@ __global__ __launch_bounds__(DN_WG) void k_dn_chunk(DnArgs a, DnScratch s) {
 #pragma unroll
         for (int u = 0; u < 4; u++) {                  // rows past the chunk are zeros
             const int t = t0 + 16 * u;
-            const float4 qg = scale4(r2[u], qk_expf_tab(gcs[t], etab));
+            const float4 qg = scale4(r2[u], qk_expf_tab(gcs[t], etab), kd - 4 * c);
             *reinterpret_cast<float4 *>(s.qg + ro + t * DN_D + 4 * c) = qg;
         }
         const float *Af = reinterpret_cast<const float *>(A);
@@ -407,8 +414,8 @@ __global__ __launch_bounds__(DN_WG) void k_dn_chunk(DnArgs a, DnScratch s) {
     bool fin = true;
 #pragma unroll
     for (int u = 0; u < 4; u++) {
-        if (part == 0) r2[u] = scale4(r2[u], bt[u]);   // V * beta
-        else r2[u] = scale4(kr[u], qk_expf_tab(gcs[t0 + 16 * u], etab));   // K * beta * exp(gcs)
+        if (part == 0) r2[u] = scale4(r2[u], bt[u], odim - 4 * c);   // V * beta
+        else r2[u] = scale4(kr[u], qk_expf_tab(gcs[t0 + 16 * u], etab), kd - 4 * c);   // K * beta * exp(gcs)
         A[(t0 + 16 * u) * (DN_D / 4) + c] = r2[u];     // plain rows: the apply reads along a row
         fin = fin && finite4(r2[u]);
     }

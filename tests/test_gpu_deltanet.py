@@ -113,16 +113,24 @@ def test_deltanet_ragged_head_dims(lib, orc):
 
 
 @pytest.mark.parametrize("H,kd,vd,n_tok", [(1, 1, 1, 1), (8, 7, 127, 65), (3, 127, 3, 63), (2, 100, 128, 129),
-                                           (24, 96, 64, 70), (8, 128, 120, 2)])
-@pytest.mark.parametrize("special", ["", "v", "k", "state"])
+                                           (24, 96, 64, 70), (8, 128, 120, 2), (3, 90, 30, 2)])
+@pytest.mark.parametrize("special", ["", "v", "k", "state", "g", "beta"])
 def test_deltanet_splits(lib, orc, H, kd, vd, n_tok, special):
     """The edges of the kernels' splits: head dims that the wide loads and
     the 16-element blocks do not divide, heads with and without the XCD
-    order, chunks of one token and one past a chunk; and the factors whose
-    zero coefficients the reference skips, infinite or NaN."""
+    order, chunks of one token and one past a chunk; the factors whose zero
+    coefficients the reference skips, infinite or NaN; and infinite scales
+    (gates that overflow, beta), which must leave the padding alone."""
     step(f"deltanet splits H={H} kd={kd} vd={vd} n={n_tok} special={special}")
     q, k, v, g, b = ssm_inputs(n_tok, H=H, kd=kd, vd=vd, seed=H * kd + n_tok, zero_rows=n_tok > 3)
     st = state0(H, kd, vd, kd)
+    if special in ("g", "beta"):                       # at the last tokens, signs so that no two infinities cancel
+        k[-2:], q[-2:], v[-2:], st = 0.1, 0.1, -np.abs(v[-2:]) - 0.1, np.abs(st) + 0.1
+    if special == "g" and n_tok > 1:                   # exp of the sum overflows at the last token but one only
+        g[:], g[-2], g[-1] = 0.0, 89.0, -29.0
+        k[-2, :, 0], k[-1], k[-1, :, 0], q[-1], q[-1, :, 0] = 0.001, 0.01, 1.0, -0.1, 10.0
+    if special == "beta":
+        b[-1] = np.inf
     bad = {"v": v, "k": k, "state": st}.get(special)
     if bad is not None:
         flat = bad.reshape(-1)
