@@ -442,9 +442,9 @@ __global__ __launch_bounds__(DN_WG) void k_dn_chunk(DnArgs a, DnScratch s) {
     else dn_apply(at, M, lane, (n + 7) / 8, o);
     float *dst = (part == 0 ? s.veff : s.kcd) + ro;
 #pragma unroll
-    for (int m = 0; m < 8; m++) {
-        dst[(wave + 8 * m) * DN_D + lane] = o[m][0];
-        dst[(wave + 8 * m) * DN_D + 64 + lane] = o[m][1];
+    for (int m = 0; m < 8; m++) {                      // an infinite attn makes the padding's sums NaN
+        dst[(wave + 8 * m) * DN_D + lane] = lane < odim ? o[m][0] : 0.0f;
+        dst[(wave + 8 * m) * DN_D + 64 + lane] = 64 + lane < odim ? o[m][1] : 0.0f;
     }
 }
 

@@ -113,14 +113,16 @@ def test_deltanet_ragged_head_dims(lib, orc):
 
 
 @pytest.mark.parametrize("H,kd,vd,n_tok", [(1, 1, 1, 1), (8, 7, 127, 65), (3, 127, 3, 63), (2, 100, 128, 129),
-                                           (24, 96, 64, 70), (8, 128, 120, 2), (3, 90, 30, 2)])
-@pytest.mark.parametrize("special", ["", "v", "k", "state", "g", "beta"])
+                                           (24, 96, 64, 70), (8, 128, 120, 2), (3, 90, 30, 2),
+                                           (3, 90, 30, 3), (2, 100, 64, 131)])
+@pytest.mark.parametrize("special", ["", "v", "k", "state", "g", "beta", "solve"])
 def test_deltanet_splits(lib, orc, H, kd, vd, n_tok, special):
     """The edges of the kernels' splits: head dims that the wide loads and
     the 16-element blocks do not divide, heads with and without the XCD
     order, chunks of one token and one past a chunk; the factors whose zero
     coefficients the reference skips, infinite or NaN; and infinite scales
-    (gates that overflow, beta), which must leave the padding alone."""
+    (gates that overflow, beta) and an infinite element of the solved matrix
+    from finite inputs, which must leave the padding alone."""
     step(f"deltanet splits H={H} kd={kd} vd={vd} n={n_tok} special={special}")
     q, k, v, g, b = ssm_inputs(n_tok, H=H, kd=kd, vd=vd, seed=H * kd + n_tok, zero_rows=n_tok > 3)
     st = state0(H, kd, vd, kd)
@@ -131,6 +133,10 @@ def test_deltanet_splits(lib, orc, H, kd, vd, n_tok, special):
         k[-2, :, 0], k[-1], k[-1, :, 0], q[-1], q[-1, :, 0] = 0.001, 0.01, 1.0, -0.1, 10.0
     if special == "beta":
         b[-1] = np.inf
+    overflows = special == "solve" and (n_tok - 1) % 64 >= 2
+    if overflows:                                      # L[i][i-1] * L[i-1][i-2] at the last token; zeros before
+        k[:], q[:], v[:], g[:], b[:], st[:] = 0.0, 0.0, 0.0, -0.1, 0.9, 1e-12
+        k[-3:], q[-3:], v[-3:] = np.sqrt(9e19 / kd), 1e-12, -0.5
     bad = {"v": v, "k": k, "state": st}.get(special)
     if bad is not None:
         flat = bad.reshape(-1)
@@ -139,6 +145,8 @@ def test_deltanet_splits(lib, orc, H, kd, vd, n_tok, special):
         flat[0] = -np.inf
     with np.errstate(all="ignore"):
         want_o, want_s = orc.deltanet_chunked(q, k, v, g, b, st)
+    if overflows:                                      # what the last row must be
+        assert np.isneginf(want_o[-1]).all() and np.isneginf(want_s).all()
     dst = dev(st)
     out = lib.deltanet_chunked(dev(q), dev(k), dev(v), dev(g), dev(b), dst)
     assert_bits_equal(host(out), want_o, "out")
