@@ -140,6 +140,81 @@ def test_add_rmsnorm_chain_splits(lib, orc, k):
     assert_bits_equal(host(xo), want_x, f"chain splits k={k}")
 
 
+def rounding_rows(k, rng):
+    """Rows whose chain rounds at almost every add: outliers among ordinary
+    values, wide and log-normal values, squares that end half a unit below
+    the sum's last place (ties, which the sum's parity decides), one binade
+    crossed per term, and sums of 0, infinity and NaN within a block."""
+    def normal():
+        return rng.standard_normal(k)
+
+    outlier = normal()
+    outlier[::400] = 3000.0
+    ties = rng.uniform(1.0, 1.41, k)
+    ties[0] = 2.0 ** 15                                # sum 2^30: an ulp of it is two of a square in [1, 2)
+    late = ties.copy()
+    late[0], late[k // 2] = 1.0, 2.0 ** 15
+    rising = np.exp2(0.5 * (np.arange(k) % 256) - 60)  # a binade a term
+    zeros = normal()
+    zeros[: k - k // 3] = 0.0
+    tiny = normal() * 2.0 ** -70                       # subnormal squares
+    tiny[-1] = 1.0
+    rows = [outlier, normal() * np.exp2(rng.integers(-28, 29, k)), np.exp(2 * normal()), ties, late, rising,
+            rising[::-1], zeros, tiny, np.zeros(k)]
+    for v in (np.inf, np.nan):
+        bad = outlier.copy()
+        bad[k // 2] = v
+        rows.append(bad)
+    both = outlier.copy()
+    both[k // 3], both[k - 1 - k // 3] = np.inf, np.nan
+    return np.asarray(rows + [both], np.float32)
+
+
+@pytest.mark.parametrize("k", [4, 8, 252, 256, 260, 512, 1024, 2560, 4096, 4100, 8196, 16384])
+def test_add_rmsnorm_rounding_rows(lib, orc, k):
+    step(f"add_rmsnorm rounding rows k={k}")
+    rng = np.random.default_rng(k + 13)
+    for delta_scale in (0.0, 1e-3):
+        h = rounding_rows(k, rng)
+        delta = (delta_scale * rng.standard_normal(h.shape)).astype(np.float32)
+        w = (1 + 0.02 * rng.standard_normal(k)).astype(np.float32)
+        ho, xo = empty(h.shape), empty(h.shape)
+        lib.add_rmsnorm_q8k(dev(h), dev(delta), dev(w), 1e-6, h_out=ho, x_out=xo)
+        want_r, want_x = orc.add_rmsnorm(h, delta, w, 1e-6)
+        assert_bits_equal(host(ho), want_r, "h + delta")
+        assert_bits_equal(host(xo), want_x, f"rounding rows k={k}")
+
+
+def test_add_rmsnorm_time_of_outlier_rows(lib):
+    """Rows whose sums round throughout (outliers in a residual stream) may
+    take longer than Gaussian rows, but not in proportion to the roundings:
+    at most 10 times at the widest row (term by term on one lane: 6 times;
+    one pass per guess found wrong: 40 times)."""
+    import torch
+    step("add_rmsnorm time of outlier rows k=16384")
+    rng = np.random.default_rng(3)
+    k = 16384
+    plain = rng.standard_normal((1, k)).astype(np.float32)
+    outlier = plain.copy()
+    outlier[:, ::400] = 3000.0
+    w, xo = dev(np.ones(k, np.float32)), empty((1, k))
+
+    def best(h):
+        hd, times = dev(h), []
+        for _ in range(10):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(50):
+                lib.add_rmsnorm_q8k(hd, None, w, 1e-6, x_out=xo)
+            b.record()
+            torch.cuda.synchronize()
+            times.append(a.elapsed_time(b))
+        return min(times)
+
+    best(plain)
+    assert best(outlier) < 10 * best(plain)
+
+
 def test_add_rmsnorm_many_scales(lib, orc):
     """4096 constant rows spanning 60 binades: as many distinct
     rscale = 1/sqrtf(mean + eps) values, each correctly rounded."""
