@@ -273,6 +273,7 @@ __global__ __launch_bounds__(DN_WG) void k_dn_chunk(DnArgs a, DnScratch s) {
             kr[u] = A[(t0 + 16 * u) * (DN_D / 4) + c];
             r2[u] = B[(t0 + 16 * u) * (DN_D / 4) + c];
         }
+        __syncthreads();                               // the same rows are written below, in another column order
     }
     float bt[4];                                       // beta of the thread's rows
 #pragma unroll
