@@ -137,8 +137,8 @@ __device__ __forceinline__ int dn_tri(int i, int j) { return i * DN_C + (j ^ ((i
 // X[k][j] goes from its lane to the column's eight by DPP; column k + 2 of L
 // is read while step k runs. Dividing by the unit diagonal returns its
 // operand unchanged (a quiet NaN included), so the division is left out.
-// xs[m]: row rg + 8m (rows of a finished slot keep adding what is above the
-// diagonal of L, which nothing reads).
+// xs[m]: row rg + 8m (rows of a finished slot keep adding what the array holds
+// from the diagonal on, which nothing reads).
 __device__ __forceinline__ void dn_solve(const float *L, int j, int rg, float (&xs)[8]) {
     float acc[8], nl[8], cf[3][8];
     auto column = [&](int k) __attribute__((always_inline)) {
@@ -149,7 +149,8 @@ __device__ __forceinline__ void dn_solve(const float *L, int j, int rg, float (&
 #pragma unroll
     for (int m = 0; m < 8; m++) {
         const int i = rg + 8 * m;
-        nl[m] = j < i ? -L[dn_tri(rg, j) + 8 * DN_C * m] : -0.0f;   // L is 0 from the diagonal on
+        // -L of a zero from the diagonal on, where the array holds what was there before
+        nl[m] = j < i ? -L[dn_tri(rg, j) + 8 * DN_C * m] : -0.0f;
         acc[m] = xs[m] = 0.0f;
     }
     column(0);
@@ -292,7 +293,7 @@ __global__ __launch_bounds__(DN_WG) void k_dn_chunk(DnArgs a, DnScratch s) {
                 run = __fadd_rn(run, lane_value(g, t + q));
                 mine = lane == t + q ? run : mine;
             }
-        gcs[lane] = mine;
+        gcs[lane] = lane < n ? mine : 0.0f;            // exp 1 past the chunk: its rows stay zeros
         if (lane == 0) glast = run;
     }
     const int64_t ro = (int64_t)ck.slot * DN_C * DN_D; // a [64][128] (or [128][64]) array of the slot
@@ -329,7 +330,7 @@ __global__ __launch_bounds__(DN_WG) void k_dn_chunk(DnArgs a, DnScratch s) {
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const int t = tq + i;
-                e[i] = t < n ? __fmul_rn(Af[4 * dn_swz(t, d >> 2) + (d & 3)], gf[i]) : 0.0f;
+                e[i] = t < n && d < kd ? __fmul_rn(Af[4 * dn_swz(t, d >> 2) + (d & 3)], gf[i]) : 0.0f;
             }
             *reinterpret_cast<float4 *>(s.kgt + ro + d * DN_C + tq) = make_float4(e[0], e[1], e[2], e[3]);
         }
@@ -410,7 +411,7 @@ __global__ __launch_bounds__(DN_WG) void k_dn_chunk(DnArgs a, DnScratch s) {
         }
         return;
     }
-    // rows past the chunk: zeros, so that their solve and apply give zeros
+    // L's rows past the chunk: zeros, not what the array held before
     for (int p = tid; p < (DN_C - n) * DN_C; p += DN_WG) D[dn_tri(n + p / DN_C, p % DN_C)] = 0.0f;
     bool fin = true;
 #pragma unroll
@@ -444,8 +445,9 @@ __global__ __launch_bounds__(DN_WG) void k_dn_chunk(DnArgs a, DnScratch s) {
     float *dst = (part == 0 ? s.veff : s.kcd) + ro;
 #pragma unroll
     for (int m = 0; m < 8; m++) {                      // an infinite attn makes the padding's sums NaN
-        dst[(wave + 8 * m) * DN_D + lane] = lane < odim ? o[m][0] : 0.0f;
-        dst[(wave + 8 * m) * DN_D + 64 + lane] = 64 + lane < odim ? o[m][1] : 0.0f;
+        const int w = wave + 8 * m < n ? odim : 0;     // and the rows' past the chunk
+        dst[(wave + 8 * m) * DN_D + lane] = lane < w ? o[m][0] : 0.0f;
+        dst[(wave + 8 * m) * DN_D + 64 + lane] = 64 + lane < w ? o[m][1] : 0.0f;
     }
 }
 
