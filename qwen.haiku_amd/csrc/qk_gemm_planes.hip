@@ -352,6 +352,7 @@ __global__ __launch_bounds__(64 * S) void k_gemm_planes_ks(const uint8_t *__rest
     // 2^lsplit workgroups share a tile, each 32 >> lsplit of its rows: the
     // other rows' lanes read past the buffer (zeros, no memory access)
     const int64_t g = blockIdx.x >> lsplit, t0 = (int64_t)blockIdx.y * 32;
+    if (g * 32 >= n) return;                           // the grid's padding: the whole workgroup
     const bool mine = (col >> (5 - lsplit)) == (int)(blockIdx.x & ((1u << lsplit) - 1));
     const int wlane = mine ? 16 * lane : 0x40000000;
     const int mrows = (m - t0 < 32) ? (int)(m - t0) : 32;
@@ -569,25 +570,28 @@ template <int TYPE>
 static void launch_planes(const uint8_t *wp, int64_t n, int nb, const uint8_t *xq, int64_t m, float *y, int fused,
                           bool ks, hipStream_t s) {
     if (ks) {
-        // Q6_K: operands a round ahead when the tiles fit one workgroup per
-        // CU (1024 x 3584: M = 128 11.3 -> 10.4 us; Q5_K and more tiles
-        // were slower with it)
+        // Operands a round ahead when the tiles fit one workgroup per CU: Q6_K
+        // (1024 x 3584: M = 128 11.3 -> 10.4 us), and every type with eight
+        // super-blocks a round; Q5_K with four, and more tiles, were slower
+        // with it.
         dim3 grid((unsigned)((n + 31) / 32), (unsigned)((m + 31) / 32));
         const uint64_t tiles = (uint64_t)grid.x * grid.y;
         const bool pf = tiles <= 256;
         int lsplit = 0;
 #define QK_PLKS(F, S, P) \
     hipLaunchKernelGGL((k_gemm_planes_ks<TYPE, F, S, P>), grid, dim3(64 * S), 0, s, wp, n, nb, xq, m, y, lsplit)
-        // There, eight super-blocks a round where that halves the rounds or
-        // nearly so (planes from HBM: Q5_K 1024 x 2048 at M = 23 5.8 -> 5.2
-        // us, 768 x 1536 at M = 300 5.8 -> 5.2, Q6_K 2560 x 7168 at M = 33
-        // 18.4 -> 17.0; nine or ten super-blocks 6.8 -> 7.1, so not those).
-        // Beyond twelve the planes of a tile are 230 KB and more, and up to
-        // four workgroups share them, 8 rows (128-byte pieces) each, while
-        // that leaves one workgroup per CU (Q6_K 1024 x 3584: M = 23 10.4 ->
-        // 8.8 us, 128 10.3 -> 9.0, 256 10.4 -> 9.8; with few super-blocks the
-        // shared activations cost as much: 1024 x 1024 3.8 -> 3.9).
-        if (pf && nb > 4 && (nb <= 8 || nb > 12)) {
+        // There, eight super-blocks a round where that leaves at most three
+        // rounds of five (planes from HBM: Q5_K 1024 x 2048 at M = 23 5.8 ->
+        // 5.2 us, 768 x 1536 at M = 300 5.8 -> 5.2, Q6_K 2560 x 7168 at M =
+        // 33 18.4 -> 17.0; nine or ten super-blocks, two rounds of three, 6.8
+        // -> 7.1). Beyond twelve the planes of a tile are 230 KB and more, and
+        // up to four workgroups share them, 8 rows (128-byte pieces) each,
+        // while that leaves one workgroup per CU (Q6_K 1024 x 3584: M = 23
+        // 10.4 -> 8.8 us, 128 10.3 -> 9.0, 256 10.4 -> 9.8; with few
+        // super-blocks the shared activations cost as much: 1024 x 1024 3.8 ->
+        // 3.9).
+        const int rounds4 = (nb + 3) / 4, rounds8 = (nb + 7) / 8;
+        if (pf && 5 * rounds8 <= 3 * rounds4) {
             if (nb > 12) lsplit = tiles <= 64 ? 2 : tiles <= 128 ? 1 : 0;
             grid.x <<= lsplit;
             if (fused) QK_PLKS(true, 8, true);
@@ -601,6 +605,15 @@ static void launch_planes(const uint8_t *wp, int64_t n, int nb, const uint8_t *x
                 return;
             }
         }
+        // Workgroups go to the XCDs in turn, so a group's token tiles meet on
+        // one XCD only if eight divides the number of groups; with an odd
+        // number every XCD reads every group's planes. Where what an XCD reads
+        // then is more than its 4 MB of L2, the groups are padded to a multiple
+        // of eight (Q5_K 2016 x 2048 at M = 384 20.0 -> 11.8 us); below that
+        // the even shares matter more (1592 x 768 at M = 299 5.4 -> 6.8 with
+        // the padding).
+        const uint64_t share = (grid.x | 8) & -(grid.x | 8);   // 8: one XCD reads an eighth of the planes; 1: all
+        if ((uint64_t)grid.x * nb * pl_chunk(TYPE) > share << 22) grid.x = (grid.x + 7) & ~7u;
         if (fused) QK_PLKS(true, 4, false);
         else QK_PLKS(false, 4, false);
 #undef QK_PLKS
@@ -611,26 +624,36 @@ static void launch_planes(const uint8_t *wp, int64_t n, int nb, const uint8_t *x
     }
 }
 
-// Kernel choice by 32 x 32 output tiles (one MI355X, Q5_K / Q6_K shapes of
-// config 3 and the model's projections, M = 64 .. 2048): up to 1024 tiles
-// the super-blocks run across waves (k_gemm_planes_ks: Q6_K 1024 x 3584
-// at M = 512 15.1 us against 22.4 for k_gemm_planes, Q5_K 2048 x 1024 at
-// M = 512 8.3 / 12.2); beyond, 64-token tiles walk the super-blocks
-// (Q6_K at M = 2048 28.0 / 37.6, Q5_K 2048 x 1024 at M = 1024 11.0 /
-// 12.6). One token tile or four per wave were slower everywhere, eight waves
-// per tile wherever the tiles outnumber the CUs. The line moves with what
-// the last round of the first kernel's four waves leaves idle: three of
-// them with one super-block, so 768 tiles (Q5_K 6144 x 256 at M = 160 7.2
-// against 5.8 us, Q6_K 6.3 / 5.6; at 768 tiles 6.1 / 5.7 and 5.3 / 5.5);
-// none with four, so 1280 (Q5_K 4096 x 1024 at M = 290 10.8 / 12.2, Q6_K
-// 10.1 / 11.4; from 1536 equal), and Q6_K with three as well (8.3 / 9.3;
-// Q5_K 9.6 / 10.1 there but 9.4 / 9.1 at 1024 x 768, M = 1280). With two,
-// and from five on, the two meet near 1024 or within 6 % of each other.
+// Kernel choice by 32 x 32 output tiles: up to `most` of them the super-blocks
+// run across waves (k_gemm_planes_ks), beyond that 64-token tiles walk them
+// (k_gemm_planes). One token tile or four per wave were slower everywhere,
+// eight waves per tile wherever the tiles outnumber the CUs. The first kernel
+// pays a round of four super-blocks whether it is full or not, so its line
+// falls with the share of a round that is idle (down to half when three of
+// four waves are, not to a quarter: staging and sums are shared); the second
+// kernel's start and end weigh more the fewer the rounds are, and it gives
+// way more with Q6_K. Measured for Q4_K, Q5_K and Q6_K with 1 .. 28
+// super-blocks at 640 .. 1792 tiles: following this line costs 0.14 % against
+// the better kernel at each point, one line at 1024 tiles 1.6 %. Where they
+// meet (second kernel's time over the first's, Q5_K at 1024 tiles): one
+// super-block 0.76, two 0.95, three 1.11, four 1.24, five 0.90, eight 1.17,
+// nine 0.96, twelve 1.18, twenty-eight 1.18; Q6_K 0.86, 1.04, 1.18, 1.28,
+// 0.95, 1.23, 1.04, 1.24, 1.33.
+static uint64_t planes_ks_tiles(int type, int nb, uint64_t groups) {
+    const int rounds = (nb + 3) / 4;
+    uint64_t most = (uint64_t)(1050 + 275 / rounds) * (nb + 2 * rounds) / (6 * rounds);
+    if (type == 14) most += most / 4;
+    // Past 4096 rows of more than four super-blocks the planes come from memory
+    // for few token tiles each: no further than 1024 (Q6_K 8695 x 4096 at M =
+    // 126, 1088 tiles, 42.6 against 34.1 us).
+    return groups > 128 && nb > 4 && most > 1024 ? 1024 : most;
+}
+
 hipError_t launch_gemm_planes(int type, const uint8_t *wp, int64_t n, int64_t k, const uint8_t *xq, int64_t m,
                               float *y, int fused, hipStream_t s) {
     const int nb = (int)(k / QK_K);
-    const int most = nb == 1 ? 768 : nb == 4 || (nb == 3 && type == 14) ? 1280 : 1024;
-    const bool ks = (uint64_t)((n + 31) / 32) * (uint64_t)((m + 31) / 32) <= (uint64_t)most && (m + 31) / 32 <= 65535;
+    const uint64_t groups = (uint64_t)(n + 31) / 32;
+    const bool ks = groups * (uint64_t)((m + 31) / 32) <= planes_ks_tiles(type, nb, groups) && (m + 31) / 32 <= 65535;
     switch (type) {
         case 12: launch_planes<12>(wp, n, nb, xq, m, y, fused, ks, s); break;
         case 13: launch_planes<13>(wp, n, nb, xq, m, y, fused, ks, s); break;

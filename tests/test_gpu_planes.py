@@ -10,8 +10,8 @@ ragged row groups (n not a multiple of 32) and token tiles, one super-block,
 k at the limit, and blocks at the ends of their ranges (Q4_K / Q5_K scales
 and quants at their maxima, Q6_K int8 scales over the whole byte range), so
 the planes' hi digit reaches +-32 and the bsums reach their bounds. Both
-kernels are reached for every type: up to 1024 32 x 32 output tiles the
-super-blocks run across waves, beyond that 64-token tiles walk them."""
+kernels are reached for every type: with few 32 x 32 output tiles the
+super-blocks run across waves, with more 64-token tiles walk them."""
 import numpy as np
 import pytest
 
@@ -84,10 +84,17 @@ def test_matmul_planes_few_tiles(tier, orc, wtype, n, nb, m, epi, t):
 
 
 # Both sides of the line between super-blocks across waves and 64-token
-# tiles, where few super-blocks move it: 768 tiles with one, 1280 with four
-# (Q6_K: with three too).
+# tiles, which moves with the share of a round of four super-blocks that is
+# filled: 662 tiles with one super-block (Q6_K 827), 890 with five (1112),
+# 1104 with three (1380), 1325 with four (1656); at most 1024 past 128 row
+# groups with more than four super-blocks. Row groups padded to a multiple
+# of eight (41 and 223 of five, 33 of eight, 161 of three), and not.
 @pytest.mark.parametrize("n,nb,m", [(6144, 1, 100), (6150, 1, 100), (5110, 3, 250), (5130, 3, 250), (8190, 4, 130),
-                                    (8200, 4, 130)])
+                                    (8200, 4, 130), (5280, 1, 100), (5290, 1, 100), (6590, 1, 100), (6600, 1, 100),
+                                    (1270, 5, 710), (1300, 5, 700), (1270, 5, 890), (1300, 5, 890), (2200, 3, 500),
+                                    (2220, 3, 500), (1910, 3, 730), (1920, 3, 750), (1690, 4, 800), (1696, 4, 810),
+                                    (2302, 4, 736), (2304, 4, 750), (980, 3, 1050), (980, 3, 1060), (1050, 4, 300),
+                                    (1050, 8, 300), (4100, 8, 224), (4100, 8, 256)])
 @pytest.mark.parametrize("wtype", [13, 14])
 def test_matmul_planes_few_super_blocks(tier, orc, wtype, n, nb, m):
     lib, k = tier, 256 * nb
