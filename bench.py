@@ -641,8 +641,9 @@ def e2e(prompt=512, gen=256, seed=0, timeout=600):
         if isinstance(out.get(cname), dict):
             out[cname]["cores"] = 1
             out[cname].pop("host_syncs_per_token", None)
-    out["tokens_identical"] = all(out[g]["tokens_identical"] for g, _ in pairs
-                                  if isinstance(out.get(g), dict) and "tokens_identical" in out[g])
+    # None (null): a pair was not compared, since its programs are not built
+    same = [out[g].get("tokens_identical") if isinstance(out[g], dict) else None for g, _ in pairs]
+    out["tokens_identical"] = False if False in same else None if None in same else True
     for v in out.values():
         if isinstance(v, dict):
             v.pop("tokens", None)
