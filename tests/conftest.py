@@ -29,6 +29,13 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs an MI355X (gfx950) GPU")
 
 
+def pytest_collection_modifyitems(items):
+    """test_e2e.py last: its programs are built from the reference's sources,
+    and where those are absent its failures should not keep a run with -x from
+    the other tests."""
+    items.sort(key=lambda item: item.path.name == "test_e2e.py")
+
+
 @pytest.fixture(scope="session")
 def orc():
     return oracle.Oracle()
