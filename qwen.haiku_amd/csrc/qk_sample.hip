@@ -13,14 +13,13 @@
 //  * after any prefix the slots hold the k largest values of the prefix
 //    (ties kept by the earlier element), so logit i (i >= k) enters iff
 //    fewer than k earlier logits are >= it;
-//  * per block of logits: the block's k largest values (k_smp_blocks);
-//    the k-th largest value T_b of everything before the block, by
-//    bisection over the union of those lists (held in registers, counted
-//    by ballots); then, for the block's logits above T_b, the exact count
-//    of earlier logits >= them (the earlier logits above T_b, fewer than
-//    k, plus the block's own earlier candidates). Those with a count
-//    below k are the entering events, listed in index order with their
-//    values (k_smp_events);
+//  * per block of logits: the block's k largest values, sorted
+//    (k_smp_blocks); the k largest values of everything before the block by
+//    merging those lists (in registers), the last of them T_b; then, for the
+//    block's logits above T_b, the exact count of earlier logits >= them (a
+//    search in the merged list, plus the block's own earlier candidates).
+//    Those with a count below k are the entering events, listed in index
+//    order with their values (k_smp_events);
 //  * the final slots: in closed form (past SMP_NMAX elements one wave
 //    replays the events in order on the k slots); then the rest
 //    of the chain on the k survivors as the reference writes it
