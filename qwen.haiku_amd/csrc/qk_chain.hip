@@ -34,12 +34,13 @@ __device__ __forceinline__ float silu(float v, const uint64_t *tab) {
 // guesses move by the same difference. A few such steps settle a row whose
 // sum seldom rounds (most Gaussian ones: none). Every step costs a pass over
 // the block (0.09 us), so a row that rounds often (outliers among ordinary
-// values) gets NORM_MOVES of them per block and NORM_ROUNDS over the blocks;
-// then the rest of the row is added exactly (exact_from). Rows with every
-// 400th element 3000, Gaussian else, us a launch: 1 x 1024 6, 4096 12, 16384
-// 30; by such steps alone 10, 62, 1150; by one lane, term by term, 13, 47,
-// 182. (Only rows of 256 of widely different terms take longer so than on one
-// lane: 6 to 7 us against 5.)
+// values) gets NORM_MOVES of them per block, NORM_MOVES_ON where a block moved,
+// and NORM_ROUNDS over the blocks; then the rest of the row is added exactly
+// (exact_from). One Gaussian block in 400000 needs more than ten. Rows with
+// every 400th element 3000, Gaussian else, us a launch: 1 x 1024 6, 4096 12,
+// 16384 28; by such steps alone 7 to 10, 62, 1150; by one lane, term by term,
+// 13, 47, 182. (Only rows of 256 of widely different terms take longer so than
+// on one lane: 5 to 8 us against 5.)
 template <int CTRL, int ROWS = 0xF>
 __device__ __forceinline__ double dpp64(double v) {
     const uint64_t b = (uint64_t)__double_as_longlong(v);
@@ -87,7 +88,8 @@ __device__ __forceinline__ void squares(float4 r, double (&t)[4]) {
     t[3] = (double)__fmul_rn(r.w, r.w);
 }
 
-constexpr int NORM_MOVES = 5, NORM_ROUNDS = 8;
+constexpr int NORM_WAVES = 16;                         // of a workgroup, at most
+constexpr int NORM_MOVES = 10, NORM_MOVES_ON = 4, NORM_ROUNDS = 5;
 
 // The guesses after segment f (lanes above f) once f's end is known.
 __device__ __forceinline__ double move_starts(double st, double end, int f, int lane) {
@@ -101,12 +103,12 @@ __device__ __forceinline__ double move_starts(double st, double end, int f, int 
 // st (moved on as they are found wrong). Lane 63's value is the block's end,
 // exact for lane 0's start unless a guess is still wrong: the ends are right
 // up to lane `open` then (64: all).
-__device__ __forceinline__ double check_block(double &st, const double (&t)[4], int lane, int &open) {
+__device__ __forceinline__ double check_block(double &st, const double (&t)[4], int lane, int most, int &open) {
     for (int m = 0;; m++) {
         const double e = add4(st, t), next = dpp64<0x130>(st);   // wave_shl:1, in every lane
         const uint64_t off = __ballot((lane < 63) & !same_bits(e, next));
         open = off ? (int)__builtin_ctzll(off) : 64;
-        if (__builtin_expect(off == 0 || m == NORM_MOVES, 1)) return e;
+        if (__builtin_expect(off == 0 || m == most, 1)) return e;
         st = move_starts(st, readlane64(e, open), open, lane);
     }
 }
@@ -224,8 +226,8 @@ __device__ __forceinline__ double block_exact(double s, const double (&t)[4], in
 // pairs: two doubles a block and one more. Of block `first`, the lanes below
 // `from` are known to end at `sure`.
 __device__ __forceinline__ double exact_from(const float4 *row, double *pairs, double starts, double sum, int first,
-                                             int nblk, int from, double sure) {
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), W = blockDim.x >> 6;
+                                             int nblk, int W, int from, double sure) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const bool scan = nblk - first > 1;
     double u[4];
     for (int blk = wave; blk < nblk; blk += W) {
@@ -282,17 +284,17 @@ __global__ __launch_bounds__(1024) void k_add_rmsnorm(const float *h, const floa
     __shared__ double sure[QK_NORM_MAX_K / QK_K];      // of such a block: the last end that is right,
     __shared__ int upto[QK_NORM_MAX_K / QK_K];         // and its lane
     extern __shared__ float4 row4[];                   // the row, where a guess was wrong
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), W = blockDim.x >> 6;
-    const int nblk = (k + QK_K - 1) / QK_K;
+    const int nblk = (k + QK_K - 1) / QK_K, W = NB == 1 ? nblk : NORM_WAVES;   // as launched
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t row = (int64_t)blockIdx.x * k;
     float4 r[NB], g[NB];
     {
         float4 a[NB];
 #pragma unroll
         for (int b = 0; b < NB; b++) {
-            const uint32_t i = (wave + W * b) * QK_K + 4 * lane;
+            const int i = (wave + W * b) * QK_K + 4 * lane;
             r[b] = a[b] = g[b] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (i < (uint32_t)k) {                    // k is a multiple of 4
+            if (i < k) {                              // k is a multiple of 4
                 r[b] = *reinterpret_cast<const float4 *>(h + row + i);
                 if (delta) a[b] = *reinterpret_cast<const float4 *>(delta + row + i);
                 g[b] = *reinterpret_cast<const float4 *>(w + i);
@@ -307,8 +309,8 @@ __global__ __launch_bounds__(1024) void k_add_rmsnorm(const float *h, const floa
     double t[NB][4], q[NB];
 #pragma unroll
     for (int b = 0; b < NB; b++) {
-        const uint32_t i = (wave + W * b) * QK_K + 4 * lane;
-        if (h_out && i < (uint32_t)k) *reinterpret_cast<float4 *>(h_out + row + i) = r[b];
+        const int i = (wave + W * b) * QK_K + 4 * lane;
+        if (h_out && i < k) *reinterpret_cast<float4 *>(h_out + row + i) = r[b];
         squares(r[b], t[b]);
         const double own = __dadd_rn(__dadd_rn(t[b][0], t[b][1]), __dadd_rn(t[b][2], t[b][3]));
         const double incl = wave_scan64(own, false);
@@ -331,7 +333,7 @@ __global__ __launch_bounds__(1024) void k_add_rmsnorm(const float *h, const floa
             const int blk = wave + W * b;
             if (blk < nblk) {
                 int open;
-                const double e = check_block(q[b], t[b], lane, open);
+                const double e = check_block(q[b], t[b], lane, round == 0 ? NORM_MOVES : NORM_MOVES_ON, open);
                 if (__builtin_expect(open == 64, 1)) {
                     if (lane == 63) ends[blk] = e;
                 } else if (lane == open) {
@@ -373,7 +375,7 @@ __global__ __launch_bounds__(1024) void k_add_rmsnorm(const float *h, const floa
         for (int b = 0; b < NB; b++)
             if (wave + W * b < nblk) row4[(wave + W * b) * 64 + lane] = r[b];
         const bool open = ends[first] == -1.0;
-        ssq = exact_from(row4, pairs, starts, ssq, first, nblk, open ? upto[first] + 1 : 0, sure[first]);
+        ssq = exact_from(row4, pairs, starts, ssq, first, nblk, W, open ? upto[first] + 1 : 0, sure[first]);
     }
     // ssq / k; for a power of two the product with 1 / k is the same value
     const double mean = (k & (k - 1)) == 0 ? __dmul_rn(ssq, 1.0 / (double)k) : __ddiv_rn(ssq, (double)k);
@@ -382,14 +384,13 @@ __global__ __launch_bounds__(1024) void k_add_rmsnorm(const float *h, const floa
     const float rscale = __fdiv_rn(1.0f, __builtin_sqrtf(__fadd_rn(__double2float_rn(mean), eps)));
 #pragma unroll
     for (int b = 0; b < NB; b++) {
-        const int blk = wave + W * b;
-        const uint32_t i = blk * QK_K + 4 * lane;
+        const int blk = wave + W * b, i = blk * QK_K + 4 * lane;
         if (blk >= nblk) break;                       // whole wave
         const float e[4] = {__fmul_rn(__fmul_rn(r[b].x, rscale), g[b].x),
                             __fmul_rn(__fmul_rn(r[b].y, rscale), g[b].y),
                             __fmul_rn(__fmul_rn(r[b].z, rscale), g[b].z),
                             __fmul_rn(__fmul_rn(r[b].w, rscale), g[b].w)};
-        if (x_out && i < (uint32_t)k) *reinterpret_cast<float4 *>(x_out + row + i) = make_float4(e[0], e[1], e[2], e[3]);
+        if (x_out && i < k) *reinterpret_cast<float4 *>(x_out + row + i) = make_float4(e[0], e[1], e[2], e[3]);
         if (xq) {                                     // k % 256 == 0: every lane is in range
             uint32_t packed, bs;
             float d;
@@ -449,8 +450,8 @@ __global__ __launch_bounds__(256) void k_swiglu(const float *__restrict__ gate, 
 // up to 1024 threads go out in several launches.
 hipError_t launch_add_rmsnorm(const float *h, const float *delta, const float *w, float eps, int64_t m, int64_t k,
                               float *h_out, float *x_out, uint8_t *xq, hipStream_t s) {
-    const int nblk = (int)((k + QK_K - 1) / QK_K), waves = nblk < 16 ? nblk : 16;
-    auto kernel = nblk <= 16 ? k_add_rmsnorm<1> : nblk <= 32 ? k_add_rmsnorm<2> : k_add_rmsnorm<4>;
+    const int nblk = (int)((k + QK_K - 1) / QK_K), waves = nblk < NORM_WAVES ? nblk : NORM_WAVES;
+    auto kernel = nblk <= NORM_WAVES ? k_add_rmsnorm<1> : nblk <= 2 * NORM_WAVES ? k_add_rmsnorm<2> : k_add_rmsnorm<4>;
     const int64_t rows = (int64_t)1 << 21;
     for (int64_t t = 0; t < m; t += rows) {
         const unsigned grid = (unsigned)(m - t < rows ? m - t : rows);
