@@ -609,7 +609,7 @@ static void launch_planes(const uint8_t *wp, int64_t n, int nb, const uint8_t *x
         // one XCD only if eight divides the number of groups; with an odd
         // number every XCD reads every group's planes. Where what an XCD reads
         // then is more than its 4 MB of L2, the groups are padded to a multiple
-        // of eight (Q5_K 2016 x 2048 at M = 384 20.0 -> 11.8 us); below that
+        // of eight (Q5_K 2016 x 2048 at M = 384 19.2 -> 11.1 us); below that
         // the even shares matter more (1592 x 768 at M = 299 5.4 -> 6.8 with
         // the padding).
         const uint64_t share = (grid.x | 8) & -(grid.x | 8);   // 8: one XCD reads an eighth of the planes; 1: all
